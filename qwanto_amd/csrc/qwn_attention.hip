@@ -21,6 +21,7 @@
 //     flattened kv_head*head_dim channels (the reference's grouping).
 #include "qwn_device.h"
 #include "qwn_internal.h"
+#include "qwn_kv.h"
 
 #include <algorithm>
 
@@ -30,40 +31,10 @@ namespace {
 constexpr int kAttnThreads = 256;
 constexpr int kMaxSplitTokens = 256;
 
-// Each KV head's pages are contiguous, so a workgroup streaming one head's
-// span of the context reads one contiguous run of keys and one of values.
-// key byte of (token, head, channel); channels 16q .. 16q + 15 of a token
-// are the 16 bytes at k_index(token, head, 16q)
-__device__ __forceinline__ size_t k_index(const KvCache &c, uint32_t token, uint32_t head, uint32_t dim) {
-    const uint32_t page = token / kKvPageTokens, slot = token % kKvPageTokens;
-    const uint32_t chunks = (c.head_dim + 15) / 16;
-    return (((static_cast<size_t>(head) * c.pages + page) * chunks + dim / 16) * kKvPageTokens + slot) * 16 +
-           dim % 16;
-}
-
-// value byte of (token, head, channel)
-__device__ __forceinline__ size_t v_offset(const KvCache &c, uint32_t token, uint32_t head, uint32_t dim) {
-    const uint32_t page = token / kKvPageTokens, slot = token % kKvPageTokens;
-    return ((static_cast<size_t>(head) * c.pages + page) * c.head_dim + dim) * kKvPageTokens + slot;
-}
-
-// the 16 value bytes of (page, head, channel)
-__device__ __forceinline__ size_t v_page_offset(const KvCache &c, uint32_t page, uint32_t head, uint32_t dim) {
-    return ((static_cast<size_t>(head) * c.pages + page) * c.head_dim + dim) * kKvPageTokens;
-}
-
 __device__ __forceinline__ void store_q8(const KvCache &c, bool is_v, uint32_t token, uint32_t head, uint32_t dim,
                                          int8_t q) {
     if (is_v) c.values[v_offset(c, token, head, dim)] = q;
     else c.keys[k_index(c, token, head, dim)] = q;
-}
-
-// scale of (token, group): [group][64-token quad][slot 0..15][page of the
-// quad 0..3], so the four floats at scale_index(64q + slot, g) are the
-// scales of tokens slot, 16 + slot, 32 + slot, 48 + slot of quad q
-__device__ __forceinline__ size_t scale_index(const KvCache &c, uint32_t token, uint32_t group) {
-    return ((static_cast<size_t>(group) * c.quads + token / (4 * kKvPageTokens)) * kKvPageTokens +
-            token % kKvPageTokens) * 4 + (token / kKvPageTokens) % 4;
 }
 
 // grid (groups, 2, tokens): y = 0 quantizes K, y = 1 quantizes V; z is the
@@ -532,19 +503,6 @@ struct DecodeAttnArgs {
     const uint64_t *tree_mask;
     const int32_t *tree_base;
 };
-
-// Whether slot t is attended under a tree mask relative to slot `base`
-// (no tree: tree_bits() gives all ones).  The 64-bit test is a lookup of
-// the mask's two halves by the slot's offset, written without any shift by
-// a wrapped offset: an earlier form, t < base || (mask >> min(t - base,
-// 63)) & 1, was compiled into the shift alone (the t < base test dropped),
-// which masked every token.
-__device__ __forceinline__ bool tree_attends(uint32_t t, uint32_t base, uint64_t mask) {
-    const uint32_t off = t - base;  // the slot's tree index when t >= base
-    const uint32_t half = off < 32u ? static_cast<uint32_t>(mask) : static_cast<uint32_t>(mask >> 32);
-    const bool bit = ((half >> (off & 31u)) & 1u) != 0u;
-    return t < base || (off < 64u && bit);
-}
 
 __device__ __forceinline__ int8_t q8_of(float x, float scale) {
     if (!isfinite(x)) return 0;
@@ -1051,8 +1009,6 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const float *__restri
 // max, sum, output), and the waves merge through LDS.
 // With one split the workgroup writes the output, else (max, sum, output)
 // partials for decode_merge_kernel.
-typedef int att_v4i __attribute__((ext_vector_type(4)));
-
 struct MfmaAttnArgs {
     KvCache c;
     const float *query;       // [H][D]
@@ -1090,26 +1046,6 @@ __device__ __forceinline__ float pieces_dot(att_v4i cacc, float s1) {
     return fmaf(s3, static_cast<float>(cacc[2]), fmaf(s2, static_cast<float>(cacc[1]), s1 * static_cast<float>(cacc[0])));
 }
 
-// Reductions over each 16-lane row by DPP row rotations (row_ror 8, 4, 2,
-// 1): every lane of the row ends with the row's max / sum (the sum's
-// association differs between lanes; callers read one lane).
-template <int CTRL>
-__device__ __forceinline__ float dpp_rot(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float row16_max(float v) {
-    v = fmaxf(v, dpp_rot<0x128>(v));
-    v = fmaxf(v, dpp_rot<0x124>(v));
-    v = fmaxf(v, dpp_rot<0x122>(v));
-    return fmaxf(v, dpp_rot<0x121>(v));
-}
-__device__ __forceinline__ float row16_sum(float v) {
-    v += dpp_rot<0x128>(v);
-    v += dpp_rot<0x124>(v);
-    v += dpp_rot<0x122>(v);
-    return v + dpp_rot<0x121>(v);
-}
-
 // DPP quad permutations: quad_perm<ctrl> moves within each 4-lane quad
 // (0xb1: lane ^ 1, 0x4e: lane ^ 2); quad_bcast_u32(v, q) gives every lane of
 // the quad lane q's v.
@@ -1125,16 +1061,6 @@ __device__ __forceinline__ uint32_t quad_bcast_u32(uint32_t v, int q) {
     case 2: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0xaa, 0xf, 0xf, false));
     default: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0xff, 0xf, 0xf, false));
     }
-}
-
-__device__ __forceinline__ float f4_at(const float4 &v, int i) {
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
-__device__ __forceinline__ void lds_wave_sync() {
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 constexpr uint32_t kMfmaMaxSplits = 512;
@@ -1578,6 +1504,18 @@ size_t mfma_attention_workspace_floats(const KvCache &c, uint32_t query_heads, u
     return nsplit > 1 ? static_cast<size_t>(query_heads) * nsplit * (c.head_dim + 2) : 0;
 }
 
+hipError_t launch_attention_merge(const float *partials, float *output, uint32_t rows, uint32_t nsplit, uint32_t D,
+                                  hipStream_t stream) {
+    const uint32_t parts = D <= 256 ? 256 / D : 0;
+    if (nsplit <= 8 * parts)
+        hipLaunchKernelGGL(decode_merge_kernel<8>, dim3(rows), dim3(256), 0, stream, partials, output, nsplit, D);
+    else if (nsplit <= 16 * parts)
+        hipLaunchKernelGGL(decode_merge_kernel<16>, dim3(rows), dim3(256), 0, stream, partials, output, nsplit, D);
+    else
+        hipLaunchKernelGGL(decode_merge_kernel<0>, dim3(rows), dim3(256), 0, stream, partials, output, nsplit, D);
+    return hipGetLastError();
+}
+
 hipError_t launch_mfma_attention(const KvCache &c, const float *query, float *output, float *partials,
                                  uint32_t query_heads, uint32_t position, const int32_t *position_ptr,
                                  uint32_t span, float scale, hipStream_t stream, const uint64_t *tree_mask,
@@ -1607,18 +1545,7 @@ hipError_t launch_mfma_attention(const KvCache &c, const float *query, float *ou
     default: e = launch_mfma_attention_rt<256>(args, plan.waves, stream); break;
     }
     if (e != hipSuccess || args.nsplit == 1) return e;
-    const uint32_t D = c.head_dim;
-    const uint32_t parts = D <= 256 ? 256 / D : 0;
-    if (args.nsplit <= 8 * parts)
-        hipLaunchKernelGGL(decode_merge_kernel<8>, dim3(query_heads), dim3(256), 0, stream, partials, output,
-                           args.nsplit, D);
-    else if (args.nsplit <= 16 * parts)
-        hipLaunchKernelGGL(decode_merge_kernel<16>, dim3(query_heads), dim3(256), 0, stream, partials, output,
-                           args.nsplit, D);
-    else
-        hipLaunchKernelGGL(decode_merge_kernel<0>, dim3(query_heads), dim3(256), 0, stream, partials, output,
-                           args.nsplit, D);
-    return hipGetLastError();
+    return launch_attention_merge(partials, output, query_heads, args.nsplit, c.head_dim, stream);
 }
 
 hipError_t launch_decode_attention(const DecodeAttentionLaunch &l, hipStream_t stream) {

@@ -204,6 +204,7 @@ struct Decoder {
     uint32_t launches = 0;
     uint32_t layer_launches = 0;  // kernels per layer
     bool fused_attention = false; // RoPE + append + attention in one kernel
+    bool block_attention = false; // a block's attention in one launch (qwn_block_attention.hip)
     uint64_t weight_bytes = 0;
 };
 
@@ -374,7 +375,29 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
             (e = launch_rope_append(d->caches[l], d->pq, d->heads, d->pk, d->pv, d->cos_tab, d->sin_tab, d->ppos, s,
                                     m, qn, kn, d->eps, tree ? d->tree_pos + row0 : nullptr)) != hipSuccess)
             return e;
-        if (d->fused_attention) {
+        // contexts past the one-split decode kernel: the block's tokens in one
+        // launch.  (One launch per token, each with its merge, took 12 us a
+        // token and layer: a 1003-token prompt through two Qwen2-1.5B layers
+        // 23.5 ms, 2.6 ms now.)  Short contexts keep the decode kernel: at 8
+        // tokens over 203 it takes 7.0 us, this one 12.3 (its sixteen-row tile
+        // is one long chain per wave).
+        if (d->block_attention && !d->fused_attention) {
+            BlockAttentionLaunch at;
+            at.cache = &d->caches[l];
+            at.query = d->pq;
+            at.output = d->pattn;
+            at.partials = d->partials;
+            at.query_heads = d->heads;
+            at.count = m;
+            at.position_ptr = d->ppos;
+            at.span = d->max_ctx;
+            at.scale = d->attn_scale;
+            if (tree) {
+                at.tree_mask = d->tree_mask + row0;
+                at.tree_base = d->tree_base;
+            }
+            if ((e = launch_block_attention(at, s)) != hipSuccess) return e;
+        } else if (d->fused_attention) {
             DecodeAttentionLaunch at;
             at.cache = &d->caches[l];
             at.query = d->pq;
@@ -757,10 +780,14 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *handle, const 
     // shape allows) and its merge
     d->fused_attention = decode_attention_supported(proto, d->heads) && d->head_dim % 64 == 0 &&
                          decode_split_tokens(proto, d->max_ctx) >= d->max_ctx;
-    part(reinterpret_cast<void **>(&d->partials),
-         std::max<size_t>(d->fused_attention ? decode_attention_workspace_floats(proto, d->heads, d->max_ctx)
-                                             : attention_at_workspace_floats(proto, d->heads),
-                          1) * 4);
+    d->block_attention = block_attention_supported(proto, d->heads);
+    size_t partials = std::max<size_t>(d->fused_attention
+                                           ? decode_attention_workspace_floats(proto, d->heads, d->max_ctx)
+                                           : attention_at_workspace_floats(proto, d->heads),
+                                       1);
+    for (uint32_t m = 1; d->block_attention && m <= d->block_tokens; ++m)
+        partials = std::max(partials, block_attention_workspace_floats(proto, d->heads, m, d->max_ctx));
+    part(reinterpret_cast<void **>(&d->partials), partials * 4);
     {
         // the head launch's shape; its buffers are not placed yet, so
         // non-null placeholders stand in for them (validity only)

@@ -402,6 +402,34 @@ uint32_t decode_split_tokens(const KvCache &c, uint32_t tokens);
 size_t decode_attention_workspace_floats(const KvCache &c, uint32_t query_heads, uint32_t tokens);
 hipError_t launch_decode_attention(const DecodeAttentionLaunch &l, hipStream_t stream);
 
+// Merges the split partials [rows][nsplit][D + 2] (max, sum, output) into
+// output [rows][D].
+hipError_t launch_attention_merge(const float *partials, float *output, uint32_t rows, uint32_t nsplit, uint32_t D,
+                                  hipStream_t stream);
+
+// Causal attention of a block of query tokens (qwn_block_attention.hip):
+// query and output [count][query_heads][head_dim], token i at cache slot
+// position_ptr[i] (device), its key and value already appended, attending to
+// slots [0, position_ptr[i]] (tree_mask / tree_base as in
+// DecodeAttentionLaunch).  span: an upper bound of the positions + 1, from
+// which the split plan and the size of partials follow.
+struct BlockAttentionLaunch {
+    const KvCache *cache = nullptr;
+    const float *query = nullptr;
+    float *output = nullptr;
+    float *partials = nullptr;   // block_attention_workspace_floats()
+    uint32_t query_heads = 0;
+    uint32_t count = 0;
+    const int32_t *position_ptr = nullptr;
+    uint32_t span = 0;
+    float scale = 1.0f;
+    const uint64_t *tree_mask = nullptr;
+    const int32_t *tree_base = nullptr;
+};
+bool block_attention_supported(const KvCache &c, uint32_t query_heads);
+size_t block_attention_workspace_floats(const KvCache &c, uint32_t query_heads, uint32_t count, uint32_t span);
+hipError_t launch_block_attention(const BlockAttentionLaunch &l, hipStream_t stream);
+
 // Device-position variants for graph replay: the token index / position is
 // read from device memory when the kernels run; attention uses a fixed grid
 // of kDevicePositionSplit-token splits over the whole cache, splits past

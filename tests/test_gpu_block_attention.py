@@ -1,0 +1,77 @@
+"""Attention of a block of tokens over a long context (qwn_block_attention.hip)
+through the resident decoder's prefill, chain verify and tree verify at
+contexts past the one-split decode kernel: row tiles of sixteen (token, head)
+pairs that end inside a token, one-row tiles, split contexts and their merge,
+every head dim, more query heads per KV head than the one-token kernels take.
+The logits are held to the oracle's rounding envelope (parity.py)."""
+import numpy as np
+import pytest
+
+from parity import oracle_envelope, step_errors, within_envelope
+from qwanto_amd import abi, synth
+
+pytestmark = pytest.mark.gpu
+
+SEEDS = tuple(range(1, 9))
+
+
+def config(heads, kv_heads, head_dim, max_ctx=1500):
+    return dict(hidden=256, intermediate=512, layers=2, heads=heads, kv_heads=kv_heads, head_dim=head_dim, vocab=1000,
+                max_ctx=max_ctx, rope_theta=1e6, rms_eps=1e-6)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,prompt,draft,qk", [
+    (6, 1, 128, 1, 2, False),      # one token: a tile of six rows
+    (6, 2, 128, 67, 11, False),    # three rows a token: tiles end inside a token
+    (4, 4, 64, 130, 16, True),     # one head per KV head: sixteen tokens a tile
+    (2, 1, 256, 40, 5, False),     # head_dim 256: keys and values loaded at their use
+    (12, 1, 64, 35, 7, False),     # more than eight heads per KV head
+    (4, 2, 64, 700, 3, False),     # 703 tokens in two splits and a merge
+    (1, 1, 128, 1300, 4, True),
+])
+def test_prefill_and_verify_match_oracle(gpu_ctx, oracle_lib, heads, kv_heads, head_dim, prompt, draft, qk):
+    rng = np.random.default_rng(heads * 1000 + head_dim + prompt)
+    cfg = config(heads, kv_heads, head_dim)
+    model = synth.decoder_model(rng, cfg, "q4_0", qk_norm=qk)
+    ids = synth.prompt_tokens(rng, cfg["vocab"], prompt + draft)
+    dec = abi.ResidentDecoder(gpu_ctx, model)
+    ref = oracle_lib.decoder(model)
+    try:
+        refs = [ref.forward(int(t)) for t in ids]
+        last, _ = dec.prefill(ids[:prompt])
+        rows, _ = dec.verify(ids[prompt:])
+    finally:
+        dec.close()
+        ref.close()
+    env = oracle_envelope(oracle_lib, model, ids, refs, SEEDS)[:, prompt - 1:]
+    ok, msg = within_envelope(step_errors([last, *rows], refs[prompt - 1:]), env)
+    assert ok, msg
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(6, 2, 128), (2, 1, 256)])
+def test_tree_matches_oracle_paths(gpu_ctx, oracle_lib, heads, kv_heads, head_dim):
+    """A tree whose siblings must not see each other, 20 nodes over a 90-token prefix."""
+    rng = np.random.default_rng(heads + head_dim)
+    cfg = config(heads, kv_heads, head_dim)
+    model = synth.decoder_model(rng, cfg, "q4_0")
+    prompt = synth.prompt_tokens(rng, cfg["vocab"], 90)
+    tokens = synth.prompt_tokens(rng, cfg["vocab"], 20)
+    parents = np.array([-1, -1] + [int(rng.integers(0, i)) for i in range(2, 20)], dtype=np.int32)
+    dec = abi.ResidentDecoder(gpu_ctx, model)
+    try:
+        dec.prefill(prompt)
+        rows, _ = dec.verify_tree(tokens, parents)
+    finally:
+        dec.close()
+    for i in (0, 1, 7, 19):
+        path, n = [], i
+        while n >= 0:
+            path.append(n)
+            n = int(parents[n])
+        ids = [int(t) for t in prompt] + [int(tokens[n]) for n in reversed(path)]
+        ref = oracle_lib.decoder(model)
+        refs = [ref.forward(t) for t in ids]
+        ref.close()
+        env = oracle_envelope(oracle_lib, model, ids, refs, SEEDS)[:, -1:]
+        ok, msg = within_envelope(step_errors([rows[i]], refs[-1:]), env)
+        assert ok, f"node {i}: {msg}"
