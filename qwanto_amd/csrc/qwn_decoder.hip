@@ -37,6 +37,7 @@ namespace {
 constexpr int kProj = 7;
 constexpr uint32_t kPrefillTokens = 16;  // tokens of a chain verify block (the GEMV's widest launch)
 constexpr uint32_t kBlockTokens = 64;    // tokens of a prompt / draft-tree block (MFMA GEMMs of 16-token groups)
+constexpr uint32_t kWideTokens = 1024;  // tokens of a prompt block on the wide GEMM
 constexpr uint32_t kTreeNodes = 64;      // draft-tree nodes per verify (c/qwanto_jetspec.h:17)
 constexpr uint32_t kTreeBlocks = kTreeNodes / kPrefillTokens;  // blocks of the narrowest block size
 enum { P_Q, P_K, P_V, P_O, P_GATE, P_UP, P_DOWN };
@@ -187,6 +188,10 @@ struct Decoder {
     uint32_t vimg_stride = 0;
     // one graph per (block size, block kind: inner / ends the prompt / verify)
     uint32_t block_tokens = kPrefillTokens;
+    // prompts of more than block_tokens tokens: blocks of up to wide_tokens
+    // on the wide GEMM (0: a projection has no MFMA-order copy, or the block
+    // attention does not take the shape), launched without a graph
+    uint32_t wide_tokens = 0;
     hipGraphExec_t prefill_exec[kBlockTokens + 1][3] = {};
     bool prefill_tried[kBlockTokens + 1][3] = {};
     // draft trees: per node its ancestor-or-self mask and rotation position
@@ -327,7 +332,8 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
     // (mode: fp32 / RMSNorm / SwiGLU of x), then the batched dot8 GEMV on
     // activation images, or where mfma_batch() says so the int8 MFMA GEMM
     // on the MFMA image; add: residual stream
-    const bool mfma = d->pmimg && mfma_batch(d->proj[P_Q]->kind, m, d->proj[P_Q]->mfma_payload != nullptr);
+    const bool wide = m > d->block_tokens;
+    const bool mfma = wide || (d->pmimg && mfma_batch(d->proj[P_Q]->kind, m, d->proj[P_Q]->mfma_payload != nullptr));
     // swiglu (MFMA, gate/up with the MFMA-order copy): outs[0] = silu(gate) * up
     auto project = [&](std::initializer_list<const DeviceTensor *> ts, std::initializer_list<float *> outs,
                        uint32_t mode, const float *x, const float *x2, const float *norm, uint32_t x_stride,
@@ -341,7 +347,7 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
         hipError_t e2;
         if (mfma) {
             if ((e2 = launch_prepare_image(t0, mode, x, x2, norm, d->eps, m, x_stride, nullptr, 0, d->pscales,
-                                           nullptr, 0, s, d->pmimg)) != hipSuccess)
+                                           nullptr, 0, s, d->pmimg, wide)) != hipSuccess)
                 return e2;
             const DeviceTensor *tv[kMaxGroup];
             float *ov[kMaxGroup];
@@ -349,6 +355,7 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
             for (const DeviceTensor *t : ts) tv[n++] = t;
             n = 0;
             for (float *o : outs) ov[n++] = o;
+            if (wide) return launch_wide_gemm(tv, ov, n, d->pmimg, d->pscales, m, nullptr, s, add, bv, swiglu);
             return launch_gemm_mfma_group(tv, ov, n, d->pmimg, d->pscales, m, nullptr, s, add, nullptr, bv, swiglu);
         }
         if ((e2 = launch_prepare_image(t0, mode, x, x2, norm, d->eps, m, x_stride, d->pimg, d->pimg_stride,
@@ -381,7 +388,7 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
         // 23.5 ms, 2.6 ms now.)  Short contexts keep the decode kernel: at 8
         // tokens over 203 it takes 7.0 us, this one 12.3 (its sixteen-row tile
         // is one long chain per wave).
-        if (d->block_attention && !d->fused_attention) {
+        if (d->block_attention && (wide || !d->fused_attention)) {
             BlockAttentionLaunch at;
             at.cache = &d->caches[l];
             at.query = d->pq;
@@ -572,12 +579,25 @@ hipError_t run_captured(hipStream_t s, hipGraphExec_t *exec, bool *tried, F enqu
     return enqueue();
 }
 
+// Tokens of the next prompt block with `left` tokens to go: a wide block
+// where the decoder has them and more than one narrow block is left.
+uint32_t prefill_block(const Decoder *d, uint32_t left) {
+    return std::min(left > d->block_tokens ? std::max(d->wide_tokens, d->block_tokens) : d->block_tokens, left);
+}
+
 // The prompt, already in feed at the device position, in prefill blocks.
 hipError_t run_prefill(Decoder *d, uint32_t count) {
     hipStream_t s = d->ctx->stream;
-    for (uint32_t i = 0; i < count; i += d->block_tokens) {
-        const uint32_t m = std::min(d->block_tokens, count - i);
+    for (uint32_t i = 0, m; i < count; i += m) {
+        m = prefill_block(d, count - i);
         const uint32_t kind = i + m == count ? kBlockLast : kBlockInner;
+        // a wide block's kernels are long enough to launch one by one; a
+        // graph for every prompt length would be kept for the decoder's life
+        if (m > d->block_tokens) {
+            const hipError_t e = enqueue_prefill(d, m, kind, s);
+            if (e != hipSuccess) return e;
+            continue;
+        }
         const hipError_t e = run_captured(s, &d->prefill_exec[m][kind], &d->prefill_tried[m][kind],
                                           [&] { return enqueue_prefill(d, m, kind, s); });
         if (e != hipSuccess) return e;
@@ -731,8 +751,17 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *handle, const 
     part(reinterpret_cast<void **>(&d->feed), static_cast<size_t>(d->max_ctx) * 4);
     part(reinterpret_cast<void **>(&d->out_tokens), static_cast<size_t>(d->max_ctx) * 4);
     // prefill blocks: [token][...] activations, images of the widest input
+    KvCache proto;
+    proto.max_tokens = d->max_ctx;
+    proto.kv_heads = d->kv_heads;
+    proto.head_dim = d->head_dim;
+    d->block_attention = block_attention_supported(proto, d->heads);
+    bool copies = true;
+    for (const DeviceTensor *t : d->proj) copies = copies && wide_gemm_supported(*t);
+    if (copies && d->block_attention) d->wide_tokens = std::min(kWideTokens, (d->max_ctx + 15) & ~15u);
+    if (d->wide_tokens <= kBlockTokens) d->wide_tokens = 0;
     {
-        const size_t P = kBlockTokens;
+        const size_t P = std::max(kBlockTokens, d->wide_tokens);
         part(reinterpret_cast<void **>(&d->px), P * D * 4);
         part(reinterpret_cast<void **>(&d->pq), P * Q * 4);
         part(reinterpret_cast<void **>(&d->pk), P * KV * 4);
@@ -749,43 +778,40 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *handle, const 
         part(reinterpret_cast<void **>(&d->pimg), kPrefillTokens * d->pimg_stride);
         // MFMA images: one per 16-token group of a block
         if (kind == kHvsq2 || kind == kQ4_0) {
-            part(reinterpret_cast<void **>(&d->pmimg),
-                 (kBlockTokens / 16) * std::max({mfma_image_bytes(*d->proj[P_DOWN]), mfma_image_bytes(*d->proj[P_Q]),
-                                                 mfma_image_bytes(*d->proj[P_O])}));
+            size_t mimg = 0;
+            for (int p : {P_Q, P_O, P_DOWN})
+                mimg = std::max({mimg, (kBlockTokens / 16) * mfma_image_bytes(*d->proj[p]),
+                                 (d->wide_tokens / 16) * wide_image_bytes(*d->proj[p])});
+            part(reinterpret_cast<void **>(&d->pmimg), mimg);
             d->block_tokens = kBlockTokens;
         }
         d->vimg_stride =
             static_cast<uint32_t>((image_bytes(d->head->kind, d->head->units) + 15) & ~static_cast<size_t>(15));
-        part(reinterpret_cast<void **>(&d->vimg), P * d->vimg_stride);
+        part(reinterpret_cast<void **>(&d->vimg), kBlockTokens * d->vimg_stride);
         if (mfma_head_supported(*d->head)) {
             part(reinterpret_cast<void **>(&d->hpieces), head_pieces_bytes_32(*d->head));
-            part(reinterpret_cast<void **>(&d->hunscale), P * 4);
+            part(reinterpret_cast<void **>(&d->hunscale), kBlockTokens * 4);
         }
         part(reinterpret_cast<void **>(&d->vlogits), static_cast<size_t>(kTreeNodes) * d->vocab * 4);
         part(reinterpret_cast<void **>(&d->vids), kTreeNodes * 4);
-        part(reinterpret_cast<void **>(&d->row_keys), P * rows_argmax_parts(d->vocab) * 8);
+        part(reinterpret_cast<void **>(&d->row_keys), kBlockTokens * rows_argmax_parts(d->vocab) * 8);
         part(reinterpret_cast<void **>(&d->tree_mask), kTreeNodes * 8);
         part(reinterpret_cast<void **>(&d->tree_pos), kTreeNodes * 4);
         part(reinterpret_cast<void **>(&d->tree_base), 4);
         part(reinterpret_cast<void **>(&d->tree_path), kTreeNodes * 4);
     }
     // attention partials of the device-position kernels
-    KvCache proto;
-    proto.max_tokens = d->max_ctx;
-    proto.kv_heads = d->kv_heads;
-    proto.head_dim = d->head_dim;
     const size_t cache_bytes = (kv_cache_layout(proto, nullptr) + 255) & ~static_cast<size_t>(255);
     // contexts of one split: RoPE, append and attention in one kernel; longer
     // ones: the RoPE/append kernel, then the split attention (MFMA where the
     // shape allows) and its merge
     d->fused_attention = decode_attention_supported(proto, d->heads) && d->head_dim % 64 == 0 &&
                          decode_split_tokens(proto, d->max_ctx) >= d->max_ctx;
-    d->block_attention = block_attention_supported(proto, d->heads);
     size_t partials = std::max<size_t>(d->fused_attention
                                            ? decode_attention_workspace_floats(proto, d->heads, d->max_ctx)
                                            : attention_at_workspace_floats(proto, d->heads),
                                        1);
-    for (uint32_t m = 1; d->block_attention && m <= d->block_tokens; ++m)
+    for (uint32_t m = 1; d->block_attention && m <= std::max(d->block_tokens, d->wide_tokens); ++m)
         partials = std::max(partials, block_attention_workspace_floats(proto, d->heads, m, d->max_ctx));
     part(reinterpret_cast<void **>(&d->partials), partials * 4);
     {
@@ -1046,7 +1072,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_prefill(QwnCudaContextHandle *handle, QwnHi
     if (e != hipSuccess) return hip_fail("decoder prefill", e);
     d->position += count;
     if (next_token) *next_token = st[0];
-    const uint64_t blocks = (count + d->block_tokens - 1) / d->block_tokens;
+    uint64_t blocks = 0;
+    for (uint32_t i = 0; i < count; ++blocks) i += prefill_block(d, count - i);
     ctx->telemetry.gpu_matmul_count += blocks * 4ull * d->layers + 1;
     return QWN_CUDA_STATUS_OK;
 }
@@ -1167,7 +1194,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_verify_tree(QwnCudaContextHandle *handle, Q
     d->tree_nodes = count;
     d->tree_parents.assign(parents, parents + count);
     d->tree_tokens.assign(tokens, tokens + count);
-    const uint64_t blocks = (count + d->block_tokens - 1) / d->block_tokens;
+    uint64_t blocks = 0;
+    for (uint32_t i = 0; i < count; ++blocks) i += prefill_block(d, count - i);
     ctx->telemetry.gpu_matmul_count += blocks * (4ull * d->layers + 1);
     return QWN_CUDA_STATUS_OK;
 }

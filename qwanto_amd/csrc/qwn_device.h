@@ -85,6 +85,16 @@ __device__ __forceinline__ void lds_barrier() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
+// Separately rounded product and sum (never contracted into an fma).
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+__device__ __forceinline__ float add_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a + b;
+}
+
 // Whole-wave sum / max, returned to every lane (row reductions by DPP, then
 // the four row totals read as scalars and combined in row order).
 __device__ __forceinline__ float wave_sum_all(float v) {

@@ -166,7 +166,8 @@ __global__ __launch_bounds__(NT) void quantize_image_kernel(const float *__restr
                                                               uint32_t q8_stride, uint32_t mode,
                                                               const float *__restrict__ x2,
                                                               const float *__restrict__ norm, float eps,
-                                                              uint32_t staged, uint8_t *mimg, size_t mimg_group) {
+                                                              uint32_t staged, uint8_t *mimg, size_t mimg_group,
+                                                              uint32_t wide) {
     extern __shared__ float vals[];  // [K] when staged
     __shared__ float wave_red[2][1024 / kWaveSize];
     constexpr uint32_t E = fused_sub_elems(KIND);
@@ -273,7 +274,20 @@ __global__ __launch_bounds__(NT) void quantize_image_kernel(const float *__restr
             if constexpr (KIND == kQ4_0) {
                 // slot (block sb/4, group sb%4): elements {0,2,4,6} then {1,3,5,7}
                 const uint32_t nblk = (K + 31) / 32;
-                if (sb < nblk * 4) {
+                if (wide) {
+                    // the wide GEMM's f16 image, 16 bytes a slot: elements
+                    // {0, 4}, {1, 5}, {2, 6}, {3, 7}; zeros to the unit's end
+                    if (sb < nsub) {
+                        uint32_t o[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            o[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(
+                                                                    static_cast<float>(static_cast<int8_t>(qb[i])),
+                                                                    static_cast<float>(static_cast<int8_t>(qb[4 + i]))));
+                        *reinterpret_cast<uint4 *>(mimg + (static_cast<size_t>(sb) * 16 + tc) * 16) =
+                            make_uint4(o[0], o[1], o[2], o[3]);
+                    }
+                } else if (sb < nblk * 4) {
                     // bytes 0, 2 / 1, 3 of each word (v_perm_b32: bytes 0-3 of
                     // the second operand, 4-7 of the first)
                     const uint32_t lo = __builtin_amdgcn_perm(w[1], w[0], 0x06040200u);
@@ -412,16 +426,6 @@ struct GemvArgs {
     const float *bias[kMaxGroup];       // per job: null, or [rows] added to the product
     uint32_t bf16;                      // kF16 layout holding bfloat16 weights
 };
-
-// Separately rounded product and sum (never contracted into an fma).
-__device__ __forceinline__ float mul_rounded(float a, float b) {
-#pragma clang fp contract(off)
-    return a * b;
-}
-__device__ __forceinline__ float add_rounded(float a, float b) {
-#pragma clang fp contract(off)
-    return a + b;
-}
 
 // Workgroup reductions for the fused prologue: every thread gets the same
 // result, combined in wave order (identical in every workgroup).
@@ -2589,11 +2593,11 @@ hipError_t launch_quantize_image(const DeviceTensor &t, const float *x, uint32_t
 hipError_t launch_prepare_image(const DeviceTensor &t, uint32_t mode, const float *x, const float *x2,
                                 const float *norm, float eps, uint32_t batch, uint32_t x_stride, uint8_t *image,
                                 uint32_t image_stride, float *scales, int8_t *q8, uint32_t q8_stride,
-                                hipStream_t stream, uint8_t *mfma_image) {
+                                hipStream_t stream, uint8_t *mfma_image, bool wide) {
     if (batch == 0 || mode > kInSwiglu || mode == kInImage || (mode == kInNorm && !norm) ||
-        (mode == kInSwiglu && !x2) || (mfma_image && batch > static_cast<uint32_t>(kMfmaMaxBatch)))
+        (mode == kInSwiglu && !x2) || (mfma_image && !wide && batch > static_cast<uint32_t>(kMfmaMaxBatch)))
         return hipErrorInvalidValue;
-    const size_t mgroup = mfma_image ? mfma_image_bytes(t) : 0;
+    const size_t mgroup = !mfma_image ? 0 : wide ? wide_image_bytes(t) : mfma_image_bytes(t);
     const uint32_t staged = static_cast<size_t>(t.cols) * sizeof(float) <= kGemvLdsLimit ? 1u : 0u;
     const size_t lds = staged ? static_cast<size_t>(t.cols) * sizeof(float) : 0;
     if (t.kind != kHvsq2 && t.kind != kQ4_0) return hipErrorInvalidValue;
@@ -2607,11 +2611,11 @@ hipError_t launch_prepare_image(const DeviceTensor &t, uint32_t mode, const floa
         if (narrow)
             hipLaunchKernelGGL((quantize_image_kernel<KD, EP, 256>), dim3(batch), dim3(256), lds, stream, x, t.cols,
                                x_stride, t.units, image, image_stride, scales, q8, q8_stride, mode, x2, norm, eps,
-                               staged, mfma_image, mgroup);
+                               staged, mfma_image, mgroup, wide ? 1u : 0u);
         else
             hipLaunchKernelGGL((quantize_image_kernel<KD, EP, 1024>), dim3(batch), dim3(1024), lds, stream, x,
                                t.cols, x_stride, t.units, image, image_stride, scales, q8, q8_stride, mode, x2, norm,
-                               eps, staged, mfma_image, mgroup);
+                               eps, staged, mfma_image, mgroup, wide ? 1u : 0u);
     };
     auto by_ept = [&](auto kind_c) {
         if (!staged) go(kind_c, std::integral_constant<int, 0>{});

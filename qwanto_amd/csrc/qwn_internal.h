@@ -203,11 +203,12 @@ hipError_t launch_gemv_group(const GemvGroupLaunch &g, hipStream_t stream);
 // Images of a block of fp32 tokens after the input transform of `mode`
 // (kInF32, kInNorm with `norm` and eps, kInSwiglu with x2 at the same
 // stride), quantized per token as launch_quantize_image; with mfma_image
-// (batch <= 16) the tokens' columns of the MFMA image are written as well.
+// (batch <= kMfmaMaxBatch) the tokens' columns of their groups' MFMA images
+// are written as well, with `wide` (any batch) those of the wide GEMM's.
 hipError_t launch_prepare_image(const DeviceTensor &t, uint32_t mode, const float *x, const float *x2,
                                 const float *norm, float eps, uint32_t batch, uint32_t x_stride, uint8_t *image,
                                 uint32_t image_stride, float *scales, int8_t *q8, uint32_t q8_stride,
-                                hipStream_t stream, uint8_t *mfma_image = nullptr);
+                                hipStream_t stream, uint8_t *mfma_image = nullptr, bool wide = false);
 // int8 MFMA batch GEMM of a HyperVSQ-2 tensor for 1..16 tokens (used from 8
 // tokens up): the activation layout its tiles read (the "MFMA image"), built
 // from int8 tokens [batch][q8_stride] (values past cols ignored), and the
@@ -230,6 +231,17 @@ hipError_t launch_gemm_mfma_group(const DeviceTensor *const *tensors, float *con
                                   const uint32_t *output_strides, hipStream_t stream, bool accumulate = false,
                                   int32_t *dump = nullptr, const float *const *biases = nullptr,
                                   bool swiglu = false);
+// The projections of a long block of tokens (qwn_wide_gemm.hip): any batch,
+// tensors with the MFMA-order copy; arguments as launch_gemm_mfma_group, the
+// image one per 16-token group of wide_image_bytes (HyperVSQ-2: the MFMA
+// image; Q4_0: the int8 activations as f16, [block][g][token 0..15][16 B],
+// elements {0,4,1,5,2,6,3,7} of the group's eight, whole units).
+size_t wide_image_bytes(const DeviceTensor &t);
+bool wide_gemm_supported(const DeviceTensor &t);
+hipError_t launch_wide_gemm(const DeviceTensor *const *tensors, float *const *outputs, uint32_t count,
+                            const uint8_t *image, const float *scales, uint32_t batch, const uint32_t *output_strides,
+                            hipStream_t stream, bool accumulate = false, const float *const *biases = nullptr,
+                            bool swiglu = false);
 constexpr uint32_t kMfmaMinTokens = 3;
 constexpr uint32_t kMfmaMinTokensQ4 = 6;
 // LDS per workgroup the MFMA GEMM plans its staging against: gfx950's
