@@ -6,10 +6,12 @@
 // workgroup of its own, so every sixteen tokens load and decode the weights
 // again and fetch their own activations: 64 tokens through one Qwen2-1.5B
 // Q4_0 layer take 34 us of GEMMs, 1003 tokens 545 us in sixteen such blocks.
-// Here a workgroup takes 128 rows x 128 tokens, its activations staged
-// through LDS once for its four waves, and the 1003 tokens take 203 us in
-// four launches (a whole prompt through two layers 2.57 -> 0.69 ms; 333
-// tokens through two Qwen3-4B HyperVSQ-2 layers 1.23 -> 0.53 ms).
+// Here a workgroup takes 64 or 128 rows x 64 tokens, its activations staged
+// through LDS once for its four waves: the 1003 tokens take 201 us in four
+// launches, and the whole prompt through two layers 0.68 ms instead of 2.57.
+// The gate/up launch (55 GFLOP, 97 us, 0.57 PFLOP/s) keeps the vector ALU
+// busy half of the time and the matrix cores a quarter: waits for a unit's
+// loads and the last, half-filled round of workgroups take the rest.
 //
 // Numerics are the sixteen-token GEMM's: exact products per weight block,
 // one fp32 multiply-add per block and output with the row's scale(s), the
@@ -36,7 +38,8 @@ typedef float wide_v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 wide_v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 wide_v8h __attribute__((ext_vector_type(8)));
 
-constexpr int kWideWaves = 4;
+constexpr int kWideWaves = 4;           // waves of a set: 16 RT rows each
+constexpr int kTokenGroups = 4;         // 16-token groups of a workgroup
 constexpr uint32_t kUnitImage = 4096;   // image bytes of one unit of a 16-token group (without the sums)
 
 struct WideArgs {
@@ -47,7 +50,7 @@ struct WideArgs {
     uint32_t rows[kMaxGroup];
     uint32_t stride[kMaxGroup];
     uint32_t job_block[kMaxGroup + 1];
-    uint32_t units, per_split;
+    uint32_t units;
     const uint8_t *image;   // one image per 16-token group
     uint32_t group_bytes;
     const float *scales;
@@ -76,14 +79,16 @@ __device__ __forceinline__ void decode_hv(const uint4 &p, uint32_t subs, wide_v4
 // 16 n in those of 1024.0 (high nibbles) give 1024 + n and 1024 + 16 n; one
 // packed f16 operation leaves n - 8, exactly.  Word order of the image:
 // elements {0, 4}, {1, 5}, {2, 6}, {3, 7} of the lane's eight.
-__device__ __forceinline__ wide_v8h decode_q4(uint32_t c) {
+// The constants in registers let the mask and the or be one instruction
+// (v_and_or_b32 takes no literal).
+__device__ __forceinline__ wide_v8h decode_q4(uint32_t c, uint32_t mlow, uint32_t mhigh, uint32_t k1024) {
     const uint32_t c8 = c >> 8;
-    auto low = [](uint32_t v) {
-        const wide_v2h h = __builtin_bit_cast(wide_v2h, (v & 0x000f000fu) | 0x64006400u);
+    auto low = [&](uint32_t v) {
+        const wide_v2h h = __builtin_bit_cast(wide_v2h, (v & mlow) | k1024);
         return h - wide_v2h{static_cast<_Float16>(1032.0f), static_cast<_Float16>(1032.0f)};
     };
-    auto high = [](uint32_t v) {
-        const wide_v2h h = __builtin_bit_cast(wide_v2h, (v & 0x00f000f0u) | 0x64006400u);
+    auto high = [&](uint32_t v) {
+        const wide_v2h h = __builtin_bit_cast(wide_v2h, (v & mhigh) | k1024);
         return __builtin_elementwise_fma(h, wide_v2h{static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)},
                                          wide_v2h{static_cast<_Float16>(-72.0f), static_cast<_Float16>(-72.0f)});
     };
@@ -91,23 +96,40 @@ __device__ __forceinline__ wide_v8h decode_q4(uint32_t c) {
     return wide_v8h{a.x, a.y, b.x, b.y, d.x, d.y, e.x, e.y};
 }
 
-// grid (row tiles of the jobs, token tiles, K splits).  A workgroup computes
+// A token group's step in the unit: its products, the operand reads of the
+// next group and the multiply-adds of the group before it (one matrix
+// instruction, then the vector instructions that run beside it).  Left to
+// itself the compiler waits out every product before its multiply-adds.
+template <int N, int V>
+__device__ __forceinline__ void interleave_steps() {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    // matrix
+        __builtin_amdgcn_sched_group_barrier(0x2, V, 0);    // vector
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// grid (row tiles of the jobs, token tiles).  A workgroup computes
 // 64 RT rows (PAIR: 32 RT rows of gate and of up) x 16 TT tokens, wave w its
 // rows 16 RT w ..: the unit's image of the workgroup's token groups is
 // staged in LDS (two buffers, the next unit's loads in flight through the
 // products, one barrier a unit), each wave's weights come straight from the
 // MFMA-order copy into registers a unit ahead.
-// SPLIT: the K split's partial sums are added to the output with float
-// atomics (accumulating launches only; in no fixed order).
-template <int KIND, int RT, int TT, bool PAIR, bool SPLIT>
-__global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs a) {
-    static_assert(!PAIR || (RT % 2 == 0 && !SPLIT), "gate/up pairs: plain stores");
+// KW > 1: KW such sets of four waves split the units, each with its own image
+// buffers; their sums meet in LDS at the end, in the sets' order.
+template <int KIND, int RT, int TT, int KW, bool PAIR>
+__global__ __launch_bounds__(64 * kWideWaves * KW, KW < 4 ? 2 : 4) void wide_gemm_kernel(WideArgs a) {
+    static_assert(!PAIR || RT % 2 == 0, "gate/up pairs: half of a wave's row groups each");
     constexpr int RO = PAIR ? RT / 2 : RT;   // row groups of output per wave
     constexpr uint32_t kStage = TT * kUnitImage;
     constexpr bool HV = KIND == kHvsq2;
-    extern __shared__ __align__(16) uint8_t smem[];   // [2][TT][4096], HV: [2][TT][64] sums
-    const uint32_t tid = threadIdx.x, lane = tid % 64;
+    constexpr uint32_t kSet = 2 * TT * (kUnitImage + (HV ? 64u : 0u));   // LDS bytes of a set's buffers
+    extern __shared__ __align__(16) uint8_t smem_all[];   // per set [2][TT][4096], HV: [2][TT][64] sums
+    const uint32_t tid = threadIdx.x % (64 * kWideWaves), lane = tid % 64;
+    const uint32_t set = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * kWideWaves));
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    uint8_t *smem = smem_all + set * kSet;
     const uint32_t g = lane >> 4, m = lane & 15;
     const uint32_t b1 = a.job_block[1], b2 = a.job_block[2], b3 = a.job_block[3];
     const uint32_t bx = blockIdx.x;
@@ -118,8 +140,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
     const uint32_t rows = a.rows[job], stride = a.stride[job], units = a.units;
     const uint32_t rg0 = ((bx - first) * kWideWaves + wave) * RO, last_rg = (rows - 1) / 16;
     const uint32_t tok0 = blockIdx.y * 16 * TT, last_grp = (a.ntok - 1) / 16;
-    const uint32_t u0 = SPLIT ? min(units, blockIdx.z * a.per_split) : 0u;
-    const uint32_t u1 = SPLIT ? min(units, u0 + a.per_split) : units;
+    // the set's units; every set runs the same number of barriers
+    const uint32_t per = (units + KW - 1) / KW;
+    const uint32_t u0 = min(units, set * per), u1 = min(units, u0 + per);
 
     // row groups past the matrix re-read the last one and store nothing
     const uint8_t *pb[RT], *mb[RT];
@@ -164,6 +187,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
         }
     };
 
+    uint32_t mlow = 0x000f000fu, mhigh = 0x00f000f0u, k1024 = 0x64006400u;
+    asm("" : "+s"(mlow), "+s"(mhigh), "+v"(k1024));
     wide_v4f acc[RT][TT];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -176,8 +201,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
         store_stage(0);
     }
     lds_barrier();
-    for (uint32_t u = u0; u < u1; ++u) {
-        const uint32_t buf = (u - u0) & 1u;
+    for (uint32_t it = 0; it < per; ++it) {
+        const uint32_t u = u0 + it, buf = it & 1u;
+        if (KW > 1 && u >= u1) {
+            lds_barrier();
+            continue;
+        }
         const uint8_t *tile = smem + buf * kStage + lane * 16;
         const uint32_t next = min(u + 1, u1 - 1);   // the last unit re-reads itself: no branch in the loop
         if constexpr (HV) {
@@ -188,10 +217,22 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
                 decode_hv(wn[i], (mn[i].y >> (8 * g)) & 0xffu, w[i]);
                 dsc[i] = half_to_float(mn[i].x & 0xffffu) * 0.125f;
                 msc[i] = half_to_float(mn[i].x >> 16);
+                asm volatile("" : "+v"(msc[i]));   // fp32 once, not in every multiply-add
             }
             load_stage(next);
             load_weights(next);
-            wide_v4i x[2][4];
+            wide_v4i x[2][4], ci[2][RT];
+            wide_v4f sa[2];
+            auto scale = [&](int t) {
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[i][t][r] =
+                            fmaf(static_cast<float>(ci[t & 1][i][r]), dsc[i], fmaf(msc[i], sa[t & 1][r], acc[i][t][r]));
+                    asm volatile("" : "+v"(acc[i][t]));
+                }
+            };
 #pragma unroll
             for (int q = 0; q < 4; ++q) x[0][q] = *reinterpret_cast<const wide_v4i *>(tile + q * 1024);
 #pragma unroll
@@ -200,24 +241,17 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
                         x[(t + 1) & 1][q] = *reinterpret_cast<const wide_v4i *>(tile + (t + 1) * kUnitImage + q * 1024);
-                const wide_v4f sa =
-                    *reinterpret_cast<const wide_v4f *>(smem + 2 * kStage + (buf * TT + t) * 64 + g * 16);
-                wide_v4i ci[RT];
+                sa[t & 1] = *reinterpret_cast<const wide_v4f *>(smem + 2 * kStage + (buf * TT + t) * 64 + g * 16);
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int i = 0; i < RT; ++i)
-                        ci[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[t & 1][q], w[i][q],
-                                                                      q ? ci[i] : wide_v4i{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < RT; ++i) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        acc[i][t][r] = fmaf(static_cast<float>(ci[i][r]), dsc[i], fmaf(msc[i], sa[r], acc[i][t][r]));
-                    asm volatile("" : "+v"(acc[i][t]));
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                        ci[t & 1][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                            x[t & 1][q], w[i][q], q ? ci[t & 1][i] : wide_v4i{0, 0, 0, 0}, 0, 0, 0);
+                if (t > 0) scale(t - 1);
+                interleave_steps<4 * RT, 3>();
             }
+            scale(TT - 1);
         } else {
             wide_v8h w[RT][4];
             float d[RT][4];
@@ -226,15 +260,25 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
                 const uint32_t cw[4] = {wn[i].x, wn[i].y, wn[i].z, wn[i].w}, dw[2] = {mn[i].x, mn[i].y};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    w[i][q] = decode_q4(cw[q]);
+                    w[i][q] = decode_q4(cw[q], mlow, mhigh, k1024);
                     d[i][q] = half_to_float((dw[q >> 1] >> (16 * (q & 1))) & 0xffffu);
+                    asm volatile("" : "+v"(d[i][q]));   // fp32 once, not in every multiply-add
                 }
             }
             load_stage(next);
             load_weights(next);
-            // a token group's operands are read while the one before it is
-            // multiplied; the barrier keeps one group's products live
             wide_v8h x[2][4];
+            wide_v4f ci[2][4][RT];
+            auto scale = [&](int t) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(ci[t & 1][q][i][r], d[i][q], acc[i][t][r]);
+#pragma unroll
+                for (int i = 0; i < RT; ++i) asm volatile("" : "+v"(acc[i][t]));
+            };
 #pragma unroll
             for (int q = 0; q < 4; ++q) x[0][q] = *reinterpret_cast<const wide_v8h *>(tile + q * 1024);
 #pragma unroll
@@ -246,27 +290,41 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
-                    for (int i = 0; i < RT; ++i) {
-                        const wide_v4f ci = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    for (int i = 0; i < RT; ++i)
+                        ci[t & 1][q][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                             x[t & 1][q], w[i][q], wide_v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[i][t][r] = fmaf(ci[r], d[i][q], acc[i][t][r]);
-                    }
-                // the group's sums are formed here: left alone, the compiler
-                // moves them behind the last product and keeps all of them live
-#pragma unroll
-                for (int i = 0; i < RT; ++i) asm volatile("" : "+v"(acc[i][t]));
-                __builtin_amdgcn_sched_barrier(0);
+                if (t > 0) scale(t - 1);
+                interleave_steps<4 * RT, 4>();
             }
+            scale(TT - 1);
         }
         // the other buffer was read a unit ago, before the last barrier
         store_stage(buf ^ 1u);
         lds_barrier();
     }
 
+    if constexpr (KW > 1) {
+        // the last barrier is behind every set's reads: the buffers are free
+        wide_v4f *part = reinterpret_cast<wide_v4f *>(smem_all) + static_cast<size_t>(wave * RT * TT) * 64 + lane;
+        constexpr uint32_t kPart = kWideWaves * RT * TT * 64;
+        if (set > 0)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) part[(set - 1) * kPart + (i * TT + t) * 64] = acc[i][t];
+        lds_barrier();
+        if (set > 0) return;
+#pragma unroll
+        for (int k = 0; k < KW - 1; ++k)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) acc[i][t] += part[k * kPart + (i * TT + t) * 64];
+    }
+
     // lane (g, m) holds tokens 4g .. 4g + 3 of row m of each tile
     float *out = a.output[job] + static_cast<size_t>(tok0 + 4 * g) * stride + rg0 * 16 + m;
-    const float *bias = PAIR || (SPLIT && blockIdx.z != 0) ? nullptr : a.bias[job];
+    const float *bias = PAIR ? nullptr : a.bias[job];
     const uint32_t row0 = rg0 * 16 + m, left = a.ntok - tok0 - min(4 * g, a.ntok - tok0);
     float bv[RO];
 #pragma unroll
@@ -289,67 +347,58 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void wide_gemm_kernel(WideArgs 
                 } else {
                     if (bias) v = add_rounded(v, bv[i]);
                 }
-                if (16u * t + r < left && row0 + 16 * i < rows) {
-                    if constexpr (SPLIT) unsafeAtomicAdd(dst, v);
-                    else *dst = !PAIR && a.accumulate ? add_rounded(*dst, v) : v;
-                }
+                if (16u * t + r < left && row0 + 16 * i < rows) *dst = !PAIR && a.accumulate ? add_rounded(*dst, v) : v;
             }
     }
 }
 
 struct WidePlan {
-    uint32_t rt = 0, tt = 0, split = 1;
+    uint32_t rt = 0, kw = 1;   // row groups per wave, sets of waves splitting K
 };
 
-template <int KIND, int RT, int TT, bool PAIR, bool SPLIT>
+template <int KIND, int RT, int TT, int KW, bool PAIR>
 hipError_t launch_wide_one(const WideArgs &a, dim3 grid, hipStream_t stream) {
-    constexpr size_t lds = 2 * TT * (kUnitImage + (KIND == kHvsq2 ? 64u : 0u));
-    hipLaunchKernelGGL((wide_gemm_kernel<KIND, RT, TT, PAIR, SPLIT>), grid, dim3(64 * kWideWaves), lds, stream, a);
+    constexpr size_t stage = KW * 2 * TT * (kUnitImage + (KIND == kHvsq2 ? 64u : 0u));
+    constexpr size_t part = (KW - 1) * kWideWaves * RT * TT * 64 * sizeof(wide_v4f);
+    constexpr size_t lds = stage > part ? stage : part;
+    static_assert(lds <= kMfmaLdsLimit, "LDS of one workgroup");
+    hipLaunchKernelGGL((wide_gemm_kernel<KIND, RT, TT, KW, PAIR>), grid, dim3(64 * kWideWaves * KW), lds, stream, a);
     return hipGetLastError();
 }
 
 template <int KIND>
 hipError_t launch_wide_kind(const WideArgs &a, const WidePlan &p, bool pair, dim3 grid, hipStream_t stream) {
-    if (pair) {
-        if (p.tt == 8) return launch_wide_one<KIND, 2, 8, true, false>(a, grid, stream);
-        return launch_wide_one<KIND, 2, 4, true, false>(a, grid, stream);
+    if (pair) return launch_wide_one<KIND, 2, kTokenGroups, 1, true>(a, grid, stream);
+    if (p.rt == 2) return launch_wide_one<KIND, 2, kTokenGroups, 1, false>(a, grid, stream);
+    switch (p.kw) {
+    case 1: return launch_wide_one<KIND, 1, kTokenGroups, 1, false>(a, grid, stream);
+    case 2: return launch_wide_one<KIND, 1, kTokenGroups, 2, false>(a, grid, stream);
+    default: return launch_wide_one<KIND, 1, kTokenGroups, 4, false>(a, grid, stream);
     }
-    if (p.split > 1) {
-        if (p.tt == 8) return launch_wide_one<KIND, 2, 8, false, true>(a, grid, stream);
-        if (p.rt == 2) return launch_wide_one<KIND, 2, 4, false, true>(a, grid, stream);
-        return launch_wide_one<KIND, 1, 4, false, true>(a, grid, stream);
-    }
-    if (p.tt == 8) return launch_wide_one<KIND, 2, 8, false, false>(a, grid, stream);
-    if (p.rt == 2) return launch_wide_one<KIND, 2, 4, false, false>(a, grid, stream);
-    return launch_wide_one<KIND, 1, 4, false, false>(a, grid, stream);
 }
 
-// Row tiles of a launch of `rt` row groups per wave (a pair's rows are one
-// matrix's).
-uint32_t wide_row_tiles(const DeviceTensor *const *tensors, uint32_t count, uint32_t out_groups) {
-    uint32_t n = 0;
-    for (uint32_t i = 0; i < count; ++i)
-        n += (tensors[i]->rows + 16 * out_groups * kWideWaves - 1) / (16 * out_groups * kWideWaves);
-    return n;
-}
-
-// Token tiles of 128 where that leaves two workgroups a CU, else of 64;
-// fewer still: a residual add splits K, a plain store halves its rows.
-WidePlan wide_plan(const DeviceTensor *const *tensors, uint32_t count, uint32_t batch, bool accumulate, bool pair) {
-    WidePlan p;
-    const uint32_t n = pair ? 1u : count;
-    auto tiles = [&](uint32_t rt, uint32_t tt) {
-        return wide_row_tiles(tensors, n, pair ? rt / 2 : rt) * ((batch + 16 * tt - 1) / (16 * tt));
+// Two row groups a wave (each operand read feeds two products) where that
+// leaves four workgroups a CU, and for the pairs; else one, and with fewer
+// than four (than one) workgroups a CU two (four) sets splitting K.  1003
+// tokens x 1536 x 8960 Q4_0 in us, groups x sets: 2x1 78, 2x2 67, 1x1 75,
+// 1x2 67, 1x4 77; 333 x 2560 x 9728 HyperVSQ-2: 47, 41, 38, 31, 30 (four K
+// splits added with float atomics: 55 and 37).  128-token tiles: 131 and 78,
+// and no faster for the pairs (1003 tokens x 2 x 8960 x 1536: 99 against 97).
+WidePlan wide_plan(const DeviceTensor *const *tensors, uint32_t count, uint32_t batch, bool pair) {
+    const uint32_t token_tiles = (batch + 16 * kTokenGroups - 1) / (16 * kTokenGroups);
+    auto tiles = [&](uint32_t rt) {
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < count; ++i) n += (tensors[i]->rows + 16 * rt * kWideWaves - 1) / (16 * rt * kWideWaves);
+        return n * token_tiles;
     };
-    p.rt = 2;
-    p.tt = tiles(2, 8) >= 2 * kChipCus ? 8 : 4;
-    if (!pair && p.tt == 4 && tiles(2, 4) < 2 * kChipCus) {
-        if (accumulate) {
-            while (p.split < 8 && tiles(2, 4) * p.split < 2 * kChipCus && tensors[0]->units >= 4 * p.split) p.split *= 2;
-        } else {
-            p.rt = 1;
-        }
+    WidePlan p;
+    if (pair || tiles(2) >= 4 * kChipCus) {
+        p.rt = 2;
+        return p;
     }
+    p.rt = 1;
+    const uint32_t sets = tiles(1) <= kChipCus ? 4 : tiles(1) < 4 * kChipCus ? 2 : 1;
+    while (p.kw < sets && tensors[0]->units >= 4 * p.kw) p.kw *= 2;
     return p;
 }
 
@@ -377,7 +426,7 @@ hipError_t launch_wide_gemm(const DeviceTensor *const *tensors, float *const *ou
     }
     if (swiglu && (count != 2 || accumulate || tensors[1]->rows != t0.rows || (biases && (biases[0] || biases[1]))))
         return hipErrorInvalidValue;
-    const WidePlan p = wide_plan(tensors, count, batch, accumulate, swiglu);
+    const WidePlan p = wide_plan(tensors, count, batch, swiglu);
     WideArgs a{};
     uint32_t grid = 0;
     const uint32_t tile_rows = 16 * kWideWaves * (swiglu ? p.rt / 2 : p.rt);
@@ -395,13 +444,12 @@ hipError_t launch_wide_gemm(const DeviceTensor *const *tensors, float *const *ou
     }
     a.job_block[kMaxGroup] = grid;
     a.units = t0.units;
-    a.per_split = (t0.units + p.split - 1) / p.split;
     a.image = image;
     a.group_bytes = static_cast<uint32_t>(wide_image_bytes(t0));
     a.scales = scales;
     a.ntok = batch;
     a.accumulate = accumulate ? 1u : 0u;
-    const dim3 dims(grid, (batch + 16 * p.tt - 1) / (16 * p.tt), p.split);
+    const dim3 dims(grid, (batch + 16 * kTokenGroups - 1) / (16 * kTokenGroups));
     return t0.kind == kHvsq2 ? launch_wide_kind<kHvsq2>(a, p, swiglu, dims, stream)
                              : launch_wide_kind<kQ4_0>(a, p, swiglu, dims, stream);
 }
