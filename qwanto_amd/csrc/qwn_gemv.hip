@@ -916,38 +916,46 @@ constexpr int kMfmaTokens = 16;
 
 __host__ __device__ constexpr size_t mfma_image_block_bytes() { return 16 * 256 + 16 * 4; }
 
+// The 16 int8 of row `src` from element e0 as four words; elements past K
+// are zero.  One 16-byte load where the row allows it.
+__device__ __forceinline__ uint4 load_q8_16(const int8_t *__restrict__ src, uint32_t e0, uint32_t K) {
+    if (e0 + 16 <= K && (reinterpret_cast<uintptr_t>(src + e0) & 15u) == 0)
+        return *reinterpret_cast<const uint4 *>(src + e0);
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i)
+        w[i >> 2] |= (e0 + i < K ? static_cast<uint32_t>(static_cast<uint8_t>(src[e0 + i])) : 0u) << (8 * (i & 3));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// One workgroup per block and 16-token group (blockIdx.y): a thread takes
+// the 16 bytes of one (slice, group, token) slot, and the block sums meet
+// over the wave's four groups by lane shuffles and over the four waves
+// (slices) in LDS.  (Summed by one thread per block and token, byte by byte,
+// the kernel took 27 us for sixteen 2560-wide tokens; 77 take 3.2 us now.)
 __global__ __launch_bounds__(256) void mfma_image_kernel(const int8_t *__restrict__ q8, uint32_t q8_stride,
-                                                         uint32_t K, uint32_t M, uint32_t units, uint8_t *img) {
-    const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < units * 256) {
-        const uint32_t m = idx % 16, g = (idx / 16) % 4, sl = (idx / 64) % 4, b = idx / 256;
-        uint32_t w[4] = {0, 0, 0, 0};
-        if (m < M) {
-            const uint32_t e0 = b * 256 + 64 * g + 16 * sl;
-            const int8_t *src = q8 + static_cast<size_t>(m) * q8_stride;
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t e = e0 + 4 * bi + k;
-                    const uint32_t v = e < K ? static_cast<uint8_t>(src[e]) : 0u;
-                    w[k] |= v << (8 * bi);
-                }
-        }
-        *reinterpret_cast<uint4 *>(img + static_cast<size_t>(idx) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    if (idx < units * 16) {
-        const uint32_t b = idx / 16, m = idx % 16;
-        int sum = 0;
-        if (m < M) {
-            const int8_t *src = q8 + static_cast<size_t>(m) * q8_stride;
-            for (uint32_t i = 0; i < 256; ++i) {
-                const uint32_t e = b * 256 + i;
-                if (e < K) sum += src[e];
-            }
-        }
-        reinterpret_cast<float *>(img + static_cast<size_t>(units) * 4096)[idx] = static_cast<float>(sum);
-    }
+                                                         uint32_t K, uint32_t M, uint32_t units, uint8_t *img,
+                                                         size_t group_bytes) {
+    __shared__ int sum_s[4][16];
+    const uint32_t tid = threadIdx.x, m = tid % 16, g = (tid / 16) % 4, sl = tid / 64, b = blockIdx.x;
+    const uint32_t token = blockIdx.y * 16 + m;
+    img += blockIdx.y * group_bytes;
+    uint4 w = make_uint4(0, 0, 0, 0);
+    if (token < M) w = load_q8_16(q8 + static_cast<size_t>(token) * q8_stride, b * 256 + 64 * g + 16 * sl, K);
+    // byte k of the four words -> word k
+    const uint32_t p01l = __builtin_amdgcn_perm(w.y, w.x, 0x05010400u), p01h = __builtin_amdgcn_perm(w.y, w.x, 0x07030602u);
+    const uint32_t p23l = __builtin_amdgcn_perm(w.w, w.z, 0x05010400u), p23h = __builtin_amdgcn_perm(w.w, w.z, 0x07030602u);
+    *reinterpret_cast<uint4 *>(img + (static_cast<size_t>(b) * 256 + tid) * 16) =
+        make_uint4(__builtin_amdgcn_perm(p23l, p01l, 0x05040100u), __builtin_amdgcn_perm(p23l, p01l, 0x07060302u),
+                   __builtin_amdgcn_perm(p23h, p01h, 0x05040100u), __builtin_amdgcn_perm(p23h, p01h, 0x07060302u));
+    int s = sdot4(w.x, 0x01010101u, sdot4(w.y, 0x01010101u, sdot4(w.z, 0x01010101u, sdot4(w.w, 0x01010101u, 0))));
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (g == 0) sum_s[sl][m] = s;
+    __syncthreads();
+    if (tid < 16)
+        reinterpret_cast<float *>(img + static_cast<size_t>(units) * 4096)[b * 16 + tid] =
+            static_cast<float>(sum_s[0][tid] + sum_s[1][tid] + sum_s[2][tid] + sum_s[3][tid]);
 }
 
 // Q4_0: one v_mfma_i32_16x16x32_i8 per 32-weight block.  A lane's weight
@@ -959,23 +967,41 @@ __global__ __launch_bounds__(256) void mfma_image_kernel(const int8_t *__restric
 //   weights need no correction).
 __host__ __device__ constexpr size_t mfma_q4_image_block_bytes() { return 4 * 16 * 8; }
 
+// WIDE: the wide GEMM's f16 image instead (elements {0,4,1,5,2,6,3,7}), to
+// the end of the last unit (nblk: whole units of four blocks).
+template <bool WIDE>
 __global__ __launch_bounds__(256) void mfma_q4_image_kernel(const int8_t *__restrict__ q8, uint32_t q8_stride,
-                                                            uint32_t K, uint32_t M, uint32_t nblk, uint8_t *img) {
+                                                            uint32_t K, uint32_t M, uint32_t nblk, uint8_t *img,
+                                                            size_t group_bytes) {
     const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < nblk * 64) {
-        const uint32_t m = idx % 16, g = (idx / 16) % 4, b = idx / 64;
-        uint32_t w[2] = {0, 0};
-        if (m < M) {
-            const int8_t *src = q8 + static_cast<size_t>(m) * q8_stride;
-            const uint32_t e0 = b * 32 + 8 * g;
+    if (idx >= nblk * 64) return;
+    const uint32_t m = idx % 16, g = (idx / 16) % 4, b = idx / 64, e0 = b * 32 + 8 * g;
+    const uint32_t token = blockIdx.y * 16 + m;
+    img += blockIdx.y * group_bytes;
+    uint2 v = make_uint2(0, 0);
+    if (token < M) {
+        const int8_t *src = q8 + static_cast<size_t>(token) * q8_stride;
+        if (e0 + 8 <= K && (reinterpret_cast<uintptr_t>(src + e0) & 7u) == 0) {
+            v = *reinterpret_cast<const uint2 *>(src + e0);
+        } else {
+            uint32_t w[2] = {0, 0};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t e = e0 + (i < 4 ? 2 * i : 2 * (i - 4) + 1);
-                const uint32_t v = e < K ? static_cast<uint8_t>(src[e]) : 0u;
-                w[i >> 2] |= v << (8 * (i & 3));
-            }
+            for (uint32_t i = 0; i < 8; ++i)
+                w[i >> 2] |= (e0 + i < K ? static_cast<uint32_t>(static_cast<uint8_t>(src[e0 + i])) : 0u) << (8 * (i & 3));
+            v = make_uint2(w[0], w[1]);
         }
-        *reinterpret_cast<uint2 *>(img + static_cast<size_t>(idx) * 8) = make_uint2(w[0], w[1]);
+    }
+    if constexpr (WIDE) {
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(
+                                                    static_cast<float>(static_cast<int8_t>((v.x >> (8 * i)) & 0xffu)),
+                                                    static_cast<float>(static_cast<int8_t>((v.y >> (8 * i)) & 0xffu))));
+        *reinterpret_cast<uint4 *>(img + static_cast<size_t>(idx) * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+        *reinterpret_cast<uint2 *>(img + static_cast<size_t>(idx) * 8) =
+            make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x06040200u), __builtin_amdgcn_perm(v.y, v.x, 0x07050301u));
     }
 }
 
@@ -2807,18 +2833,31 @@ size_t mfma_image_bytes(const DeviceTensor &t) {
 }
 
 hipError_t launch_mfma_image(const DeviceTensor &t, const int8_t *q8, uint32_t batch, uint32_t q8_stride,
-                             uint8_t *image, hipStream_t stream) {
-    if ((t.kind != kHvsq2 && t.kind != kQ4_0) || batch == 0 || batch > static_cast<uint32_t>(kMfmaTokens))
-        return hipErrorInvalidValue;
+                             uint8_t *image, hipStream_t stream, bool wide) {
+    if ((t.kind != kHvsq2 && t.kind != kQ4_0) || batch == 0) return hipErrorInvalidValue;
+    const size_t gb = wide ? wide_image_bytes(t) : mfma_image_bytes(t);
+    // a launch holds 65535 groups (grid y)
+    constexpr uint32_t kMost = 65535 * 16;
+    if (batch > kMost) {
+        const hipError_t e = launch_mfma_image(t, q8, kMost, q8_stride, image, stream, wide);
+        if (e != hipSuccess) return e;
+        return launch_mfma_image(t, q8 + static_cast<size_t>(kMost) * q8_stride, batch - kMost, q8_stride,
+                                 image + static_cast<size_t>(kMost / 16) * gb, stream, wide);
+    }
+    const uint32_t groups = (batch + 15) / 16;
     if (t.kind == kQ4_0) {
-        const uint32_t n = mfma_steps(t) * 64;
-        hipLaunchKernelGGL(mfma_q4_image_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, q8, q8_stride, t.cols,
-                           batch, mfma_steps(t), image);
+        const uint32_t nblk = wide ? 4 * t.units : mfma_steps(t);
+        const dim3 grid((nblk * 64 + 255) / 256, groups);
+        if (wide)
+            hipLaunchKernelGGL(mfma_q4_image_kernel<true>, grid, dim3(256), 0, stream, q8, q8_stride, t.cols, batch, nblk,
+                               image, gb);
+        else
+            hipLaunchKernelGGL(mfma_q4_image_kernel<false>, grid, dim3(256), 0, stream, q8, q8_stride, t.cols, batch,
+                               nblk, image, gb);
         return hipGetLastError();
     }
-    const uint32_t n = t.units * 256;
-    hipLaunchKernelGGL(mfma_image_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, q8, q8_stride, t.cols, batch,
-                       t.units, image);
+    hipLaunchKernelGGL(mfma_image_kernel, dim3(t.units, groups), dim3(256), 0, stream, q8, q8_stride, t.cols, batch,
+                       t.units, image, gb);
     return hipGetLastError();
 }
 

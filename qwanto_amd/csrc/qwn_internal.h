@@ -214,8 +214,10 @@ hipError_t launch_prepare_image(const DeviceTensor &t, uint32_t mode, const floa
 // from int8 tokens [batch][q8_stride] (values past cols ignored), and the
 // GEMM on it: output [batch][output_stride] = W x_t * scales[t].
 size_t mfma_image_bytes(const DeviceTensor &t);
+// Beyond 16 tokens: one image per 16-token group, back to back (wide: the
+// wide GEMM's).
 hipError_t launch_mfma_image(const DeviceTensor &t, const int8_t *q8, uint32_t batch, uint32_t q8_stride,
-                             uint8_t *image, hipStream_t stream);
+                             uint8_t *image, hipStream_t stream, bool wide = false);
 hipError_t launch_gemm_mfma(const DeviceTensor &t, const uint8_t *image, const float *scales, float *output,
                             uint32_t batch, uint32_t output_stride, hipStream_t stream);
 // The same over up to kMaxGroup tensors of equal K sharing one image (one

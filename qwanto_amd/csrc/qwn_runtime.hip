@@ -185,7 +185,10 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     g.output = out_dev;
     g.batch = r->batch;
     g.output_stride = r->rows;
-    const size_t mfma_img = qwn::mfma_image_bytes(t);
+    // more tokens than the 16-token GEMM takes in one launch: the wide GEMM
+    const bool wide = mfma && r->batch > static_cast<uint32_t>(qwn::kMfmaMaxBatch) && qwn::wide_gemm_supported(t);
+    const size_t group_img = wide ? qwn::wide_image_bytes(t) : qwn::mfma_image_bytes(t);
+    const size_t mfma_img = (static_cast<size_t>(r->batch) + 15) / 16 * group_img;
     if (mfma && ((e = ctx->dev_work.ensure(mfma_img + (quantize ? in_bytes / 4 : 0))) != hipSuccess))
         return hip_fail("MFMA workspace allocation", e, QWN_CUDA_STATUS_OUT_OF_MEMORY);
     (void)hipEventRecord(ctx->ev_start, ctx->stream);
@@ -201,14 +204,20 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
             q8 = dq;
         }
         uint8_t *img = static_cast<uint8_t *>(ctx->dev_work.ptr);
-        for (uint32_t t0 = 0; t0 < r->batch; t0 += 16) {
-            const uint32_t nt = std::min<uint32_t>(16, r->batch - t0);
-            if ((e = qwn::launch_mfma_image(t, q8 + static_cast<size_t>(t0) * dev_stride, nt, dev_stride, img,
-                                            ctx->stream)) != hipSuccess ||
-                (e = qwn::launch_gemm_mfma(t, img, static_cast<const float *>(ctx->dev_scales.ptr) + t0,
-                                           static_cast<float *>(ctx->dev_out.ptr) + static_cast<size_t>(t0) * r->rows,
-                                           nt, r->rows, ctx->stream)) != hipSuccess)
-                return hip_fail("MFMA GEMM launch", e);
+        if ((e = qwn::launch_mfma_image(t, q8, r->batch, dev_stride, img, ctx->stream, wide)) != hipSuccess)
+            return hip_fail("MFMA image launch", e);
+        const float *sc = static_cast<const float *>(ctx->dev_scales.ptr);
+        float *dev_out = static_cast<float *>(ctx->dev_out.ptr);
+        const qwn::DeviceTensor *ts[1] = {&t};
+        const uint32_t strides[1] = {r->rows};
+        const uint32_t step = wide ? r->batch : static_cast<uint32_t>(qwn::kMfmaMaxBatch);
+        for (uint32_t t0 = 0; t0 < r->batch; t0 += step) {
+            const uint32_t nt = std::min<uint32_t>(step, r->batch - t0);
+            float *outs[1] = {dev_out + static_cast<size_t>(t0) * r->rows};
+            e = wide ? qwn::launch_wide_gemm(ts, outs, 1, img, sc, nt, strides, ctx->stream)
+                     : qwn::launch_gemm_mfma_group(ts, outs, 1, img + (t0 / 16) * group_img, sc + t0, nt, strides,
+                                                   ctx->stream);
+            if (e != hipSuccess) return hip_fail("MFMA GEMM launch", e);
         }
     } else {
         if (quantize)

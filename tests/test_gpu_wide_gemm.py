@@ -10,6 +10,7 @@ import pytest
 
 from parity import oracle_envelope, step_errors, within_envelope
 from qwanto_amd import abi, synth
+from test_gpu_gemv import check_hvsq2, check_q4_0
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +49,18 @@ def test_wide_prefill_matches_oracle(gpu_ctx, oracle_lib, dtype, shape, prompt, 
     for got in (last, again):
         ok, msg = within_envelope(step_errors([got], refs[prompt - 1:]), env)
         assert ok, msg
+
+
+@pytest.mark.parametrize("dtype", ["q4_0", "hvsq2"])
+@pytest.mark.parametrize("N,K,M", [
+    (1, 31, 65),         # one row, K inside one unit, a one-token last group
+    (77, 777, 70),       # rows and K ending inside their tiles; four sets of waves splitting K
+    (130, 129, 40),      # 17 to 64 tokens: several groups on the 16-token GEMM
+    (2560, 1536, 160),   # two sets
+    (9000, 520, 129),    # one set
+    (17000, 256, 300),   # two row groups a wave, fewer units than sets
+])
+def test_host_batches(gpu_ctx, oracle_lib, dtype, N, K, M):
+    """qwn_cuda_abi_hypervsq2_gemm with more than 16 tokens."""
+    check = check_q4_0 if dtype == "q4_0" else check_hvsq2
+    check(gpu_ctx, oracle_lib, N, K, seed=N + K + M, M=M)
