@@ -432,7 +432,7 @@ class Context:
         if x.ndim == 1:
             x = x[None, :]
         batch, stride = x.shape
-        out = np.zeros((batch, rows), dtype=np.float32)
+        out = np.empty((batch, rows), dtype=np.float32)  # every value is written
         sc = None if scales is None else np.ascontiguousarray(scales, dtype=np.float32)
         req = GemmRequest(tensor=h, input_q8=_p(x), input_scale=float(scale or 0.0),
                           input_scales=_p(sc), output=_p(out), batch=batch, rows=rows, cols=cols,
@@ -686,7 +686,7 @@ class ResidentDecoder:
         each token [count])."""
         tokens = np.ascontiguousarray(tokens, dtype=np.int32)
         n = tokens.size
-        out = np.zeros((n, self.cfg["vocab"]), dtype=np.float32) if logits else None
+        out = np.empty((n, self.cfg["vocab"]), dtype=np.float32) if logits else None
         ids = np.zeros(n, dtype=np.int32)
         lib = self.ctx.lib
         lib.check("decoder_verify", lib.lib.qwn_hip_decoder_verify(
@@ -700,7 +700,7 @@ class ResidentDecoder:
         tokens = np.ascontiguousarray(tokens, dtype=np.int32)
         parents = np.ascontiguousarray(parents, dtype=np.int32)
         n = tokens.size
-        out = np.zeros((n, self.cfg["vocab"]), dtype=np.float32) if logits else None
+        out = np.empty((n, self.cfg["vocab"]), dtype=np.float32) if logits else None
         ids = np.zeros(n, dtype=np.int32)
         lib = self.ctx.lib
         lib.check("decoder_verify_tree", lib.lib.qwn_hip_decoder_verify_tree(
@@ -735,7 +735,7 @@ class ResidentDecoder:
 
     def forward(self, token: int, logits: bool = True):
         """One step; returns (logits or None, greedy next token)."""
-        out = np.zeros(self.cfg["vocab"], dtype=np.float32) if logits else None
+        out = np.empty(self.cfg["vocab"], dtype=np.float32) if logits else None
         nxt = ctypes.c_int32(0)
         self.ctx.lib.check("decoder_forward", self.ctx.lib.lib.qwn_hip_decoder_forward(
             self.ctx._h, ctypes.byref(self.handle), int(token), _p(out), ctypes.addressof(nxt)))
@@ -745,7 +745,7 @@ class ResidentDecoder:
         """Prompt tokens in prefill blocks; returns (last logits or None,
         greedy next token)."""
         tk = np.ascontiguousarray(tokens, dtype=np.int32)
-        out = np.zeros(self.cfg["vocab"], dtype=np.float32) if logits else None
+        out = np.empty(self.cfg["vocab"], dtype=np.float32) if logits else None
         nxt = ctypes.c_int32(0)
         self.ctx.lib.check("decoder_prefill", self.ctx.lib.lib.qwn_hip_decoder_prefill(
             self.ctx._h, ctypes.byref(self.handle), _p(tk), tk.size, _p(out), ctypes.addressof(nxt)))

@@ -75,6 +75,21 @@ struct UploadPipe {
     int next = 0;
 };
 
+// Results on their way to a caller's own (pageable) buffer: a kernel writes
+// them into pinned memory, a window at a time, and raises a flag there for
+// each piece, and the host copies a piece out while the next ones are in
+// flight.  Two windows, used in turn, so what stays pinned does not grow.
+constexpr uint32_t kDownloadPiece = 64u << 10;       // floats
+constexpr uint32_t kDownloadPieces = 4;              // of a window
+constexpr uint32_t kDownloadExtra = 64;              // words of a second, small result
+struct DownloadPipe {
+    // [2][kDownloadPieces][kDownloadPiece] floats, [2][kDownloadPieces] flags
+    // (the epoch a piece last landed in), [kDownloadExtra] words
+    PinnedBuffer data;
+    DeviceBuffer counters;  // [2][kDownloadPieces] workgroups done
+    uint32_t epoch = 0;
+};
+
 struct Context {
     std::mutex mutex;
     int device = -1;
@@ -89,6 +104,7 @@ struct Context {
     std::vector<ResidentKv *> caches;
     std::vector<Decoder *> decoders;
     UploadPipe upload;
+    DownloadPipe download;
     QwnCudaTelemetry telemetry{};
 };
 
@@ -105,6 +121,16 @@ Context *context_of(const QwnCudaContextHandle *h);
 // Handles this context issued (lock held by the caller); null otherwise.
 ResidentTensor *tensor_of(Context *ctx, const QwnCudaTensorHandle &h);
 ResidentKv *cache_of(Context *ctx, const QwnCudaKvCacheHandle &h);
+
+// Copies [rows][cols] fp32 from the device (16-byte aligned, rows back to
+// back; none when dst is null) to dst [rows][dst_stride], and `extra` words
+// (at most kDownloadExtra) to extra_dst, behind the work on the context's
+// stream, and waits for it (context lock held).
+hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const float *src, size_t cols, size_t rows,
+                         int32_t *extra_dst = nullptr, const int32_t *extra = nullptr, uint32_t extra_count = 0);
+
+// Allocates what download_rows needs (it does so itself when first called).
+hipError_t ready_download(Context *ctx);
 
 // Releases a decoder's device memory and graph (context lock held).
 void destroy_decoder(Decoder *d);

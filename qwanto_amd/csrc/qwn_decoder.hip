@@ -854,6 +854,7 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *handle, const 
     const size_t act_bytes = total;
     total += cache_bytes * d->layers;
     hipError_t e = hipSetDevice(ctx->device);
+    if (e == hipSuccess) e = ready_download(ctx);
     if (e == hipSuccess) e = hipMalloc(&d->allocation, total);
     if (e != hipSuccess) {
         delete d;
@@ -1026,11 +1027,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_forward(QwnCudaContextHandle *handle, QwnHi
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = hipMemcpyAsync(d->feed + d->position, &token, 4, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = run_step(d);
-    if (e == hipSuccess && logits)
-        e = hipMemcpyAsync(logits, d->logits, static_cast<size_t>(d->vocab) * 4, hipMemcpyDeviceToHost, s);
     int32_t st[2] = {0, 0};
-    if (e == hipSuccess) e = hipMemcpyAsync(st, d->state, sizeof(st), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = download_rows(ctx, logits, d->vocab, d->logits, d->vocab, 1, st, d->state, 2);
     if (e != hipSuccess) return hip_fail("decoder step", e);
     d->position++;
     if (next_token) *next_token = st[0];
@@ -1064,11 +1062,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_prefill(QwnCudaContextHandle *handle, QwnHi
     if (e == hipSuccess)
         e = hipMemcpyAsync(d->feed + d->position, tokens, static_cast<size_t>(count) * 4, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = run_prefill(d, count);
-    if (e == hipSuccess && logits)
-        e = hipMemcpyAsync(logits, d->logits, static_cast<size_t>(d->vocab) * 4, hipMemcpyDeviceToHost, s);
     int32_t st[2] = {0, 0};
-    if (e == hipSuccess) e = hipMemcpyAsync(st, d->state, sizeof(st), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = download_rows(ctx, logits, d->vocab, d->logits, d->vocab, 1, st, d->state, 2);
     if (e != hipSuccess) return hip_fail("decoder prefill", e);
     d->position += count;
     if (next_token) *next_token = st[0];
@@ -1103,11 +1098,9 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_verify(QwnCudaContextHandle *handle, QwnHip
     if (e == hipSuccess)
         e = hipMemcpyAsync(d->feed + d->position, tokens, static_cast<size_t>(count) * 4, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = run_verify(d, count);
-    if (e == hipSuccess && logits)
-        e = hipMemcpyAsync(logits, d->vlogits, static_cast<size_t>(count) * d->vocab * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess && next_tokens)
-        e = hipMemcpyAsync(next_tokens, d->vids, static_cast<size_t>(count) * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess)
+        e = download_rows(ctx, logits, d->vocab, d->vlogits, d->vocab, count, next_tokens, d->vids,
+                          next_tokens ? count : 0);
     if (e != hipSuccess) return hip_fail("decoder verify", e);
     d->position += count;
     ctx->telemetry.gpu_matmul_count += 4ull * d->layers + 1;
@@ -1185,17 +1178,14 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_verify_tree(QwnCudaContextHandle *handle, Q
     // the nodes stay in slots base .. base + count - 1 until a path is
     // committed; the position stays at the prefix
     if (e == hipSuccess) e = hipMemcpyAsync(d->state + 1, &base, 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && logits)
-        e = hipMemcpyAsync(logits, d->vlogits, static_cast<size_t>(count) * d->vocab * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess && next_tokens)
-        e = hipMemcpyAsync(next_tokens, d->vids, static_cast<size_t>(count) * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess)
+        e = download_rows(ctx, logits, d->vocab, d->vlogits, d->vocab, count, next_tokens, d->vids,
+                          next_tokens ? count : 0);
     if (e != hipSuccess) return hip_fail("decoder tree verify", e);
     d->tree_nodes = count;
     d->tree_parents.assign(parents, parents + count);
     d->tree_tokens.assign(tokens, tokens + count);
-    uint64_t blocks = 0;
-    for (uint32_t i = 0; i < count; ++blocks) i += prefill_block(d, count - i);
+    const uint64_t blocks = (count + d->block_tokens - 1) / d->block_tokens;
     ctx->telemetry.gpu_matmul_count += blocks * (4ull * d->layers + 1);
     return QWN_CUDA_STATUS_OK;
 }

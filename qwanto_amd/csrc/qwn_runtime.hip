@@ -64,6 +64,115 @@ ResidentKv *cache_of(Context *ctx, const QwnCudaKvCacheHandle &h) {
     return std::find(ctx->caches.begin(), ctx->caches.end(), c) != ctx->caches.end() ? c : nullptr;
 }
 
+// One window of n floats.  Bound by the link to the host.  Workgroup b copies
+// slice b % kSlices of piece b / kSlices; the last one of a piece raises its
+// flag, after every store of the piece has reached the host's memory.  A
+// runtime copy into pageable memory pins or stages it piece by piece without
+// overlap, and one into pinned memory costs about 25 us a piece with its
+// event.  One row of 151936 logits adds 36 us to a decode step instead of 66,
+// eight rows 260 us to a verify call instead of 388.
+constexpr uint32_t kSlices = 16;
+constexpr uint32_t kSlice = kDownloadPiece / kSlices;
+__global__ __launch_bounds__(256) void download_kernel(const float *__restrict__ src, float *__restrict__ dst,
+                                                       uint32_t n, const int32_t *__restrict__ extra,
+                                                       int32_t *extra_dst, uint32_t extra_count, uint32_t *counters,
+                                                       uint32_t *flags, uint32_t epoch) {
+    const uint32_t p = blockIdx.x / kSlices;
+    if (blockIdx.x == 0 && threadIdx.x < extra_count) extra_dst[threadIdx.x] = extra[threadIdx.x];
+    const uint32_t end = min(n, (blockIdx.x + 1) * kSlice);
+    for (uint32_t i = blockIdx.x * kSlice + 4 * threadIdx.x; i < end; i += 4 * blockDim.x) {
+        if (i + 4 <= end) {
+            *reinterpret_cast<float4 *>(dst + i) = *reinterpret_cast<const float4 *>(src + i);
+        } else {
+            for (uint32_t k = i; k < end; ++k) dst[k] = src[k];
+        }
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(counters + p, 1u) == kSlices - 1) {
+        counters[p] = 0;
+        __hip_atomic_store(flags + p, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+hipError_t ready_download(Context *ctx) {
+    DownloadPipe &d = ctx->download;
+    hipError_t e;
+    if (!d.data.ptr) {
+        constexpr size_t window_floats = 2 * kDownloadPieces * kDownloadPiece;
+        if ((e = d.data.ensure((window_floats + 2 * kDownloadPieces + kDownloadExtra) * sizeof(float))) != hipSuccess)
+            return e;
+        std::memset(static_cast<float *>(d.data.ptr) + window_floats, 0, 2 * kDownloadPieces * sizeof(float));
+    }
+    if (!d.counters.ptr && ((e = d.counters.ensure(2 * kDownloadPieces * 4)) != hipSuccess ||
+                            (e = hipMemsetAsync(d.counters.ptr, 0, 2 * kDownloadPieces * 4, ctx->stream)) != hipSuccess)) {
+        d.counters.release();
+        return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const float *src, size_t cols, size_t rows,
+                         int32_t *extra_dst, const int32_t *extra, uint32_t extra_count) {
+    constexpr size_t kWindow = static_cast<size_t>(kDownloadPieces) * kDownloadPiece;
+    const size_t total = dst ? cols * rows : 0, windows = std::max<size_t>(1, (total + kWindow - 1) / kWindow);
+    if (extra_count > kDownloadExtra || (dst && (reinterpret_cast<uintptr_t>(src) & 15u))) return hipErrorInvalidValue;
+    hipError_t e = ready_download(ctx);
+    if (e != hipSuccess) return e;
+    DownloadPipe &d = ctx->download;
+    auto *pinned = static_cast<float *>(d.data.ptr);
+    auto *flags = static_cast<uint32_t *>(d.data.ptr) + 2 * kWindow;
+    auto *words = static_cast<int32_t *>(d.data.ptr) + 2 * kWindow + 2 * kDownloadPieces;
+    uint32_t epochs[2] = {0, 0};
+    auto pieces = [&](size_t w) {
+        const size_t n = total - std::min(total, w * kWindow);
+        return static_cast<uint32_t>(std::max<size_t>(1, (std::min(n, kWindow) + kDownloadPiece - 1) / kDownloadPiece));
+    };
+    auto issue = [&](size_t w) {
+        const uint32_t n = static_cast<uint32_t>(std::min(kWindow, total - std::min(total, w * kWindow))), half = w & 1;
+        epochs[half] = ++d.epoch ? d.epoch : ++d.epoch;   // never the cleared flags' zero
+        hipLaunchKernelGGL(download_kernel, dim3(pieces(w) * kSlices), dim3(256), 0, ctx->stream, src + w * kWindow,
+                           pinned + half * kWindow, n, extra, words, w == 0 ? extra_count : 0u,
+                           static_cast<uint32_t *>(d.counters.ptr) + half * kDownloadPieces,
+                           flags + half * kDownloadPieces, epochs[half]);
+        return hipGetLastError();
+    };
+    if ((e = issue(0)) != hipSuccess || (windows > 1 && (e = issue(1)) != hipSuccess)) return e;
+    size_t touched = 0;
+    for (size_t w = 0; w < windows; ++w) {
+        const uint32_t half = w & 1, np = pieces(w);
+        for (uint32_t p = 0; p < np; ++p) {
+            const uint32_t *flag = flags + half * kDownloadPieces + p;
+            const size_t first = w * kWindow + static_cast<size_t>(p) * kDownloadPiece;
+            touched = std::max(touched, first);
+            // the stream is asked now and then: a failed kernel raises no flag
+            for (uint32_t spin = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != epochs[half]; ++spin) {
+                if (touched < total) {
+                    // the wait goes into the caller's pages, which a fresh
+                    // buffer does not have yet
+                    static_cast<volatile float *>(dst)[touched / cols * dst_stride + touched % cols] = 0.0f;
+                    touched += 4096 / sizeof(float);
+                }
+                __builtin_ia32_pause();
+                if (spin % 16384) continue;
+                e = hipStreamQuery(ctx->stream);
+                if (e == hipSuccess) break;
+                if (e != hipErrorNotReady) return e;
+                (void)hipGetLastError();
+            }
+            for (size_t at = first, end = std::min(total, first + kDownloadPiece); at < end;) {
+                const size_t row = at / cols, col = at % cols, n = std::min(cols - col, end - at);
+                std::memcpy(dst + row * dst_stride + col, pinned + half * kWindow + (at - w * kWindow), n * sizeof(float));
+                at += n;
+            }
+        }
+        // the window is copied out: its memory takes the one after next
+        if (w + 2 < windows && (e = issue(w + 2)) != hipSuccess) return e;
+    }
+    if (extra_count) std::memcpy(extra_dst, words, extra_count * sizeof(int32_t));
+    return hipSuccess;
+}
+
 }  // namespace qwn
 
 namespace {
@@ -136,8 +245,18 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     const size_t out_bytes = static_cast<size_t>(r->batch) * r->rows * sizeof(float);
     const uint32_t img_stride = static_cast<uint32_t>(qwn::image_bytes(t.kind, t.units));
     const size_t img_bytes = static_cast<size_t>(r->batch) * img_stride;
+    // int8 MFMA tiles of 16 tokens (mfma_batch: from 2 HyperVSQ-2 / 3 Q4_0
+    // tokens on the MFMA-order copy, from 3 / 6 without it)
+    const bool mfma = qwn::mfma_batch(t.kind, r->batch, t.mfma_payload != nullptr);
+    // Small requests skip the copy engines: the image kernel reads the
+    // activations (and the GEMV its scales) straight from the pinned staging
+    // buffer, and the GEMV epilogue stores into the pinned output buffer, so a
+    // call is two kernels and one synchronisation instead of three DMA
+    // transfers around them.  Outputs of 64K+ rows (the LM head) and the MFMA
+    // path keep the device buffers and DMA.
+    const bool zero_copy = !mfma && r->rows < 65536;
     if ((e = ctx->host_in.ensure(in_bytes + scale_bytes)) != hipSuccess ||
-        (e = ctx->host_out.ensure(out_bytes)) != hipSuccess ||
+        (e = ctx->host_out.ensure(zero_copy ? out_bytes : 0)) != hipSuccess ||
         (e = ctx->dev_in.ensure(in_bytes)) != hipSuccess ||
         (e = ctx->dev_scales.ensure(scale_bytes)) != hipSuccess ||
         (e = ctx->dev_out.ensure(out_bytes)) != hipSuccess ||
@@ -155,16 +274,6 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     }
     float *hscales = reinterpret_cast<float *>(hin + in_bytes);
     for (uint32_t b = 0; b < r->batch; ++b) hscales[b] = r->input_scales ? r->input_scales[b] : r->input_scale;
-    // int8 MFMA tiles of 16 tokens (mfma_batch: from 2 HyperVSQ-2 / 3 Q4_0
-    // tokens on the MFMA-order copy, from 3 / 6 without it)
-    const bool mfma = qwn::mfma_batch(t.kind, r->batch, t.mfma_payload != nullptr);
-    // Small requests skip the copy engines: the image kernel reads the
-    // activations (and the GEMV its scales) straight from the pinned staging
-    // buffer, and the GEMV epilogue stores into the pinned output buffer, so a
-    // call is two kernels and one synchronisation instead of three DMA
-    // transfers around them.  Outputs of 64K+ rows (the LM head) and the MFMA
-    // path keep the device buffers and DMA.
-    const bool zero_copy = !mfma && r->rows < 65536;
     if (!zero_copy &&
         ((e = hipMemcpyAsync(ctx->dev_in.ptr, hin, in_bytes, hipMemcpyHostToDevice, ctx->stream)) != hipSuccess ||
          (!quantize && (e = hipMemcpyAsync(ctx->dev_scales.ptr, hscales, scale_bytes, hipMemcpyHostToDevice,
@@ -231,16 +340,18 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
         if ((e = qwn::launch_gemv(g, ctx->stream)) != hipSuccess) return hip_fail("GEMV launch", e);
     }
     (void)hipEventRecord(ctx->ev_end, ctx->stream);
-    if (!zero_copy && (e = hipMemcpyAsync(ctx->host_out.ptr, ctx->dev_out.ptr, out_bytes, hipMemcpyDeviceToHost,
-                                          ctx->stream)) != hipSuccess)
-        return hip_fail("result download", e);
     const auto t_sync = std::chrono::steady_clock::now();
-    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return hip_fail("GEMV synchronize", e);
+    if (!zero_copy && (e = qwn::download_rows(ctx, r->output, out_stride, static_cast<const float *>(ctx->dev_out.ptr),
+                                              r->rows, r->batch)) != hipSuccess)
+        return hip_fail("result download", e);
+    if (zero_copy && (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return hip_fail("GEMV synchronize", e);
     const double sync_ms = ms_since(t_sync);
-    const float *hout = static_cast<const float *>(ctx->host_out.ptr);
-    for (uint32_t b = 0; b < r->batch; ++b)
-        std::memcpy(r->output + static_cast<size_t>(b) * out_stride, hout + static_cast<size_t>(b) * r->rows,
-                    static_cast<size_t>(r->rows) * sizeof(float));
+    if (zero_copy) {
+        const float *hout = static_cast<const float *>(ctx->host_out.ptr);
+        for (uint32_t b = 0; b < r->batch; ++b)
+            std::memcpy(r->output + static_cast<size_t>(b) * out_stride, hout + static_cast<size_t>(b) * r->rows,
+                        static_cast<size_t>(r->rows) * sizeof(float));
+    }
     float kernel_ms = 0.0f;
     if (hipEventElapsedTime(&kernel_ms, ctx->ev_start, ctx->ev_end) != hipSuccess) kernel_ms = 0.0f;
 
@@ -457,6 +568,8 @@ QWN_CUDA_ABI_API int qwn_cuda_abi_context_destroy(QwnCudaContextHandle *handle) 
         ctx->caches.clear();
         ctx->host_in.release();
         ctx->host_out.release();
+        ctx->download.data.release();
+        ctx->download.counters.release();
         ctx->dev_in.release();
         ctx->dev_out.release();
         ctx->dev_scales.release();

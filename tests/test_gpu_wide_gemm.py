@@ -64,3 +64,35 @@ def test_host_batches(gpu_ctx, oracle_lib, dtype, N, K, M):
     """qwn_cuda_abi_hypervsq2_gemm with more than 16 tokens."""
     check = check_q4_0 if dtype == "q4_0" else check_hvsq2
     check(gpu_ctx, oracle_lib, N, K, seed=N + K + M, M=M)
+
+
+@pytest.mark.parametrize("N,M", [
+    (65537, 1),      # one token past the rows that are stored to the host directly: a ragged last piece
+    (1021, 150),     # rows that pieces end inside of
+    (70003, 300),    # many windows
+])
+def test_host_results_in_pieces(gpu_ctx, oracle_lib, N, M):
+    """Results as the device wrote them, piece by piece, into rows of a larger
+    stride: every value there, the gaps untouched, twice over."""
+    import ctypes
+    rng = np.random.default_rng(N + M)
+    w = synth.q4_0_weights(rng, N, 64)
+    q8 = rng.integers(-127, 128, (M, 64), dtype=np.int8)
+    xs = np.linspace(0.5, 1.5, M, dtype=np.float32)
+    h = gpu_ctx.upload(w, "q4_0", N, 64)
+    try:
+        for _ in range(2):
+            out = np.full((M, N + 3), np.nan, dtype=np.float32)
+            req = abi.GemmRequest(tensor=h, input_q8=q8.ctypes.data, input_scale=0.0, input_scales=xs.ctypes.data,
+                                  output=out.ctypes.data, batch=M, rows=N, cols=64, input_stride=64,
+                                  output_stride=N + 3, input_mode=abi.INPUT_Q8)
+            tm = abi.Telemetry()
+            gpu_ctx.lib.check("gemm", gpu_ctx.lib.lib.qwn_cuda_abi_hypervsq2_gemm(gpu_ctx._h, ctypes.byref(req),
+                                                                                ctypes.byref(tm)))
+            assert np.isnan(out[:, N:]).all()
+            for t in sorted({0, M // 2, M - 1}):
+                ref = oracle_lib.gemv_q4_0_q8(w, q8[t], float(xs[t]), 64, N)
+                assert np.allclose(out[t, :N], ref, rtol=1e-5, atol=1e-5 * np.abs(ref).max())  # two fp32 sums of two products
+            assert not np.isnan(out[:, :N]).any()
+    finally:
+        gpu_ctx.release(h)
