@@ -11,6 +11,7 @@
 // context has its own lock.
 #include "qwn_context.h"
 #include "qwn_cuda_abi.h"
+#include "qwn_download.h"
 #include "qwn_hip_ext.h"
 #include "qwn_internal.h"
 
@@ -145,20 +146,30 @@ hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const floa
             const uint32_t *flag = flags + half * kDownloadPieces + p;
             const size_t first = w * kWindow + static_cast<size_t>(p) * kDownloadPiece;
             touched = std::max(touched, first);
-            // the stream is asked now and then: a failed kernel raises no flag
-            for (uint32_t spin = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != epochs[half]; ++spin) {
-                if (touched < total) {
-                    // the wait goes into the caller's pages, which a fresh
-                    // buffer does not have yet
-                    static_cast<volatile float *>(dst)[touched / cols * dst_stride + touched % cols] = 0.0f;
-                    touched += 4096 / sizeof(float);
-                }
-                __builtin_ia32_pause();
-                if (spin % 16384) continue;
-                e = hipStreamQuery(ctx->stream);
-                if (e == hipSuccess) break;
-                if (e != hipErrorNotReady) return e;
-                (void)hipGetLastError();
+            hipError_t failed = hipErrorLaunchFailure;
+            const Landing landing = await_piece(
+                flag, epochs[half],
+                [&] {
+                    if (touched < total) {
+                        // the wait goes into the caller's pages, which a
+                        // fresh buffer does not have yet
+                        map_for_writing(dst + touched / cols * dst_stride + touched % cols);
+                        touched += 4096 / sizeof(float);
+                    }
+                    __builtin_ia32_pause();
+                },
+                [&] {
+                    const hipError_t q = hipStreamQuery(ctx->stream);
+                    if (q == hipSuccess) return StreamState::kDone;
+                    (void)hipGetLastError();
+                    if (q == hipErrorNotReady) return StreamState::kBusy;
+                    failed = q;
+                    return StreamState::kFailed;
+                });
+            if (landing != Landing::kLanded) {
+                // a piece's count may have stopped half way: cleared before the next use
+                d.counters.release();
+                return failed;
             }
             for (size_t at = first, end = std::min(total, first + kDownloadPiece); at < end;) {
                 const size_t row = at / cols, col = at % cols, n = std::min(cols - col, end - at);
