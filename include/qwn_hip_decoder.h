@@ -91,7 +91,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_destroy(QwnCudaContextHandle *context, QwnH
 /* Empties the KV cache (position 0). */
 QWN_CUDA_ABI_API int qwn_hip_decoder_reset(QwnCudaContextHandle *context, QwnHipDecoderHandle *decoder);
 /* One step on `token` at the current position (synchronous).  `logits`
- * (vocab floats) and `next_token` (the greedy choice) may be NULL. */
+ * (vocab floats, host or GPU memory) and `next_token` (the greedy choice,
+ * host) may be NULL. */
 QWN_CUDA_ABI_API int qwn_hip_decoder_forward(QwnCudaContextHandle *context, QwnHipDecoderHandle *decoder,
                                              int32_t token, float *logits, int32_t *next_token);
 /* `count` prompt tokens at the current position in prefill blocks of up to

@@ -127,7 +127,7 @@ ResidentKv *cache_of(Context *ctx, const QwnCudaKvCacheHandle &h);
 // (at most kDownloadExtra) to extra_dst, behind the work on the context's
 // stream, and waits for it (context lock held).  Until a piece of 256 KB has
 // landed its part of dst keeps what it held; after an error the pieces that
-// landed before it are there.
+// landed before it are there.  dst and extra_dst may be GPU memory.
 hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const float *src, size_t cols, size_t rows,
                          int32_t *extra_dst = nullptr, const int32_t *extra = nullptr, uint32_t extra_count = 0);
 

@@ -113,13 +113,34 @@ hipError_t ready_download(Context *ctx) {
     return hipSuccess;
 }
 
+// Whether p is GPU memory (pinned and managed memory the host can store to).
+static bool on_device(const void *p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();   // memory the runtime does not know
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice;
+}
+
 hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const float *src, size_t cols, size_t rows,
                          int32_t *extra_dst, const int32_t *extra, uint32_t extra_count) {
     constexpr size_t kWindow = static_cast<size_t>(kDownloadPieces) * kDownloadPiece;
     const size_t total = dst ? cols * rows : 0, windows = std::max<size_t>(1, (total + kWindow - 1) / kWindow);
     if (extra_count > kDownloadExtra || (dst && (reinterpret_cast<uintptr_t>(src) & 15u))) return hipErrorInvalidValue;
-    hipError_t e = ready_download(ctx);
-    if (e != hipSuccess) return e;
+    hipError_t e;
+    if ((dst && on_device(dst)) || (extra_count && on_device(extra_dst))) {
+        // the host cannot store there: the runtime's copies (a destination on
+        // the host is told apart in about a microsecond)
+        if (dst && (e = hipMemcpy2DAsync(dst, dst_stride * sizeof(float), src, cols * sizeof(float), cols * sizeof(float),
+                                         rows, hipMemcpyDefault, ctx->stream)) != hipSuccess)
+            return e;
+        if (extra_count && (e = hipMemcpyAsync(extra_dst, extra, extra_count * sizeof(int32_t), hipMemcpyDefault,
+                                               ctx->stream)) != hipSuccess)
+            return e;
+        return hipStreamSynchronize(ctx->stream);
+    }
+    if ((e = ready_download(ctx)) != hipSuccess) return e;
     DownloadPipe &d = ctx->download;
     auto *pinned = static_cast<float *>(d.data.ptr);
     auto *flags = static_cast<uint32_t *>(d.data.ptr) + 2 * kWindow;

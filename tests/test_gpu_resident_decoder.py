@@ -364,3 +364,43 @@ def test_verify_block_matches_oracle_steps(gpu_ctx, oracle_lib, cfg, dtype, P, M
     if again is not None:
         ok, msg = within_envelope(step_errors([again], [logits[2]]), env[:, 2:3], k=2 * ENV_K)
         assert ok, "step after truncate vs verify: " + msg
+
+
+def test_logits_into_gpu_memory(gpu_ctx):
+    """Every entry point that returns logits takes GPU memory for them, and
+    verify for its ids too: the values a host buffer gets."""
+    import ctypes
+
+    import torch
+    rng = np.random.default_rng(77)
+    model = synth.decoder_model(rng, SMALL, "q4_0")
+    V, ids = SMALL["vocab"], synth.prompt_tokens(rng, SMALL["vocab"], 3)
+    parents = np.array([-1, 0, 0], dtype=np.int32)
+    dec = abi.ResidentDecoder(gpu_ctx, model)
+    lib, ctx, h = gpu_ctx.lib.lib, gpu_ctx._h, ctypes.byref(dec.handle)
+
+    def ptr(a):
+        return ctypes.c_void_p(a.data_ptr() if torch.is_tensor(a) else a.ctypes.data)
+
+    calls = {"forward": (1, lambda y, n: lib.qwn_hip_decoder_forward(ctx, h, int(ids[0]), ptr(y), None)),
+             "prefill": (1, lambda y, n: lib.qwn_hip_decoder_prefill(ctx, h, ptr(ids), 3, ptr(y), None)),
+             "verify": (3, lambda y, n: lib.qwn_hip_decoder_verify(ctx, h, ptr(ids), 3, ptr(y), ptr(n))),
+             "verify_tree": (3, lambda y, n: lib.qwn_hip_decoder_verify_tree(ctx, h, ptr(ids), ptr(parents), 3, ptr(y),
+                                                                             ptr(n)))}
+    try:
+        for name, (rows, call) in calls.items():
+            host, host_ids = np.full((rows, V), np.nan, dtype=np.float32), np.full(3, -1, dtype=np.int32)
+            dev = torch.full((rows, V), float("nan"), device="cuda:0")
+            dev_ids = torch.full((3,), -1, device="cuda:0", dtype=torch.int32)
+            torch.cuda.synchronize()
+            for y, n in ((host, host_ids), (dev, dev_ids)):
+                dec.reset()
+                gpu_ctx.lib.check(name, call(y, n))
+            got = dev.cpu().numpy()
+            # two runs of the same call: K splits added with float atomics
+            # may move an int8 activation one step, here as between two host runs
+            assert np.linalg.norm(got - host) <= 2e-2 * np.linalg.norm(host), name
+            if name.startswith("verify"):
+                assert dev_ids.cpu().tolist() == got.argmax(axis=1).tolist() and host_ids.tolist() == host.argmax(axis=1).tolist()
+    finally:
+        dec.close()
