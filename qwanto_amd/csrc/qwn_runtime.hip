@@ -384,8 +384,14 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
             std::memcpy(r->output + static_cast<size_t>(b) * out_stride, hout + static_cast<size_t>(b) * r->rows,
                         static_cast<size_t>(r->rows) * sizeof(float));
     }
+    // the results' flags say nothing of the events: the runtime gives a time
+    // only for events that it knows to be complete
     float kernel_ms = 0.0f;
-    if (hipEventElapsedTime(&kernel_ms, ctx->ev_start, ctx->ev_end) != hipSuccess) kernel_ms = 0.0f;
+    if (hipEventSynchronize(ctx->ev_end) != hipSuccess ||
+        hipEventElapsedTime(&kernel_ms, ctx->ev_start, ctx->ev_end) != hipSuccess) {
+        (void)hipGetLastError();   // not the next launch's error
+        kernel_ms = 0.0f;
+    }
 
     QwnCudaTelemetry &tm = ctx->telemetry;
     tm.gpu_matmul_count++;

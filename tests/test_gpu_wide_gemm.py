@@ -96,3 +96,20 @@ def test_host_results_in_pieces(gpu_ctx, oracle_lib, N, M):
             assert not np.isnan(out[:, :N]).any()
     finally:
         gpu_ctx.release(h)
+
+
+def test_every_call_adds_its_kernel_time(gpu_ctx):
+    """gpu_kernel_ms on the path whose results are polled for: a call that
+    adds nothing read its events before they were complete."""
+    rng = np.random.default_rng(5)
+    h = gpu_ctx.upload(synth.q4_0_weights(rng, 256, 512), "q4_0", 256, 512)
+    q8, xs = rng.integers(-127, 128, (20, 512), dtype=np.int8), np.ones(20, dtype=np.float32)
+    try:
+        ms = [gpu_ctx.telemetry().gpu_kernel_ms]
+        for _ in range(200):
+            gpu_ctx.gemm(h, q8, 256, 512, scales=xs)
+            ms.append(gpu_ctx.telemetry().gpu_kernel_ms)
+    finally:
+        gpu_ctx.release(h)
+    steps = np.diff(ms)
+    assert (steps > 0).all() and steps.max() < 100.0
