@@ -2834,16 +2834,9 @@ size_t mfma_image_bytes(const DeviceTensor &t) {
 
 hipError_t launch_mfma_image(const DeviceTensor &t, const int8_t *q8, uint32_t batch, uint32_t q8_stride,
                              uint8_t *image, hipStream_t stream, bool wide) {
-    if ((t.kind != kHvsq2 && t.kind != kQ4_0) || batch == 0) return hipErrorInvalidValue;
-    const size_t gb = wide ? wide_image_bytes(t) : mfma_image_bytes(t);
     // a launch holds 65535 groups (grid y)
-    constexpr uint32_t kMost = 65535 * 16;
-    if (batch > kMost) {
-        const hipError_t e = launch_mfma_image(t, q8, kMost, q8_stride, image, stream, wide);
-        if (e != hipSuccess) return e;
-        return launch_mfma_image(t, q8 + static_cast<size_t>(kMost) * q8_stride, batch - kMost, q8_stride,
-                                 image + static_cast<size_t>(kMost / 16) * gb, stream, wide);
-    }
+    if ((t.kind != kHvsq2 && t.kind != kQ4_0) || batch == 0 || batch > 65535u * 16) return hipErrorInvalidValue;
+    const size_t gb = wide ? wide_image_bytes(t) : mfma_image_bytes(t);
     const uint32_t groups = (batch + 15) / 16;
     if (t.kind == kQ4_0) {
         const uint32_t nblk = wide ? 4 * t.units : mfma_steps(t);

@@ -215,7 +215,7 @@ hipError_t launch_prepare_image(const DeviceTensor &t, uint32_t mode, const floa
 // GEMM on it: output [batch][output_stride] = W x_t * scales[t].
 size_t mfma_image_bytes(const DeviceTensor &t);
 // Beyond 16 tokens: one image per 16-token group, back to back (wide: the
-// wide GEMM's).
+// wide GEMM's); at most 65535 groups.
 hipError_t launch_mfma_image(const DeviceTensor &t, const int8_t *q8, uint32_t batch, uint32_t q8_stride,
                              uint8_t *image, hipStream_t stream, bool wide = false);
 hipError_t launch_gemm_mfma(const DeviceTensor &t, const uint8_t *image, const float *scales, float *output,
@@ -233,9 +233,9 @@ hipError_t launch_gemm_mfma_group(const DeviceTensor *const *tensors, float *con
                                   const uint32_t *output_strides, hipStream_t stream, bool accumulate = false,
                                   int32_t *dump = nullptr, const float *const *biases = nullptr,
                                   bool swiglu = false);
-// The projections of a long block of tokens (qwn_wide_gemm.hip): any batch,
-// tensors with the MFMA-order copy; arguments as launch_gemm_mfma_group, the
-// image one per 16-token group of wide_image_bytes (HyperVSQ-2: the MFMA
+// The projections of a long block of tokens (qwn_wide_gemm.hip; a launch holds
+// 65535 tiles of 64), tensors with the MFMA-order copy: arguments as
+// launch_gemm_mfma_group, the image one per 16-token group of wide_image_bytes (HyperVSQ-2: the MFMA
 // image; Q4_0: the int8 activations as f16, [block][g][token 0..15][16 B],
 // elements {0,4,1,5,2,6,3,7} of the group's eight, whole units).
 size_t wide_image_bytes(const DeviceTensor &t);

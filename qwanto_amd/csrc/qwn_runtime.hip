@@ -257,6 +257,11 @@ ResidentTensor *check_request(Context *ctx, const QwnCudaGemmRequest *r) {
     return rt;
 }
 
+// Tokens of a host batch whose images are held at a time (a multiple of 64):
+// 256 token tiles fill the chip whatever the rows, the images stay within
+// 0.6 GB at 19456 columns, and no launch's grid grows with the batch.
+constexpr uint32_t kImageTokens = 16384;
+
 int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *telemetry) {
     ResidentTensor *rt = check_request(ctx, r);
     if (!rt) return QWN_CUDA_STATUS_INVALID_ARGUMENT;
@@ -329,7 +334,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     // more tokens than the 16-token GEMM takes in one launch: the wide GEMM
     const bool wide = mfma && r->batch > static_cast<uint32_t>(qwn::kMfmaMaxBatch) && qwn::wide_gemm_supported(t);
     const size_t group_img = wide ? qwn::wide_image_bytes(t) : qwn::mfma_image_bytes(t);
-    const size_t mfma_img = (static_cast<size_t>(r->batch) + 15) / 16 * group_img;
+    const size_t mfma_img = (static_cast<size_t>(std::min(r->batch, kImageTokens)) + 15) / 16 * group_img;
     if (mfma && ((e = ctx->dev_work.ensure(mfma_img + (quantize ? in_bytes / 4 : 0))) != hipSuccess))
         return hip_fail("MFMA workspace allocation", e, QWN_CUDA_STATUS_OUT_OF_MEMORY);
     (void)hipEventRecord(ctx->ev_start, ctx->stream);
@@ -345,20 +350,24 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
             q8 = dq;
         }
         uint8_t *img = static_cast<uint8_t *>(ctx->dev_work.ptr);
-        if ((e = qwn::launch_mfma_image(t, q8, r->batch, dev_stride, img, ctx->stream, wide)) != hipSuccess)
-            return hip_fail("MFMA image launch", e);
         const float *sc = static_cast<const float *>(ctx->dev_scales.ptr);
         float *dev_out = static_cast<float *>(ctx->dev_out.ptr);
         const qwn::DeviceTensor *ts[1] = {&t};
         const uint32_t strides[1] = {r->rows};
-        const uint32_t step = wide ? r->batch : static_cast<uint32_t>(qwn::kMfmaMaxBatch);
-        for (uint32_t t0 = 0; t0 < r->batch; t0 += step) {
-            const uint32_t nt = std::min<uint32_t>(step, r->batch - t0);
-            float *outs[1] = {dev_out + static_cast<size_t>(t0) * r->rows};
-            e = wide ? qwn::launch_wide_gemm(ts, outs, 1, img, sc, nt, strides, ctx->stream)
-                     : qwn::launch_gemm_mfma_group(ts, outs, 1, img + (t0 / 16) * group_img, sc + t0, nt, strides,
-                                                   ctx->stream);
-            if (e != hipSuccess) return hip_fail("MFMA GEMM launch", e);
+        const uint32_t step = wide ? kImageTokens : static_cast<uint32_t>(qwn::kMfmaMaxBatch);
+        for (uint32_t i0 = 0, ni; i0 < r->batch; i0 += ni) {
+            ni = std::min(kImageTokens, r->batch - i0);
+            if ((e = qwn::launch_mfma_image(t, q8 + static_cast<size_t>(i0) * dev_stride, ni, dev_stride, img,
+                                            ctx->stream, wide)) != hipSuccess)
+                return hip_fail("MFMA image launch", e);
+            for (uint32_t t0 = 0; t0 < ni; t0 += step) {
+                const uint32_t nt = std::min(step, ni - t0);
+                float *outs[1] = {dev_out + static_cast<size_t>(i0 + t0) * r->rows};
+                e = wide ? qwn::launch_wide_gemm(ts, outs, 1, img, sc + i0, nt, strides, ctx->stream)
+                         : qwn::launch_gemm_mfma_group(ts, outs, 1, img + (t0 / 16) * group_img, sc + i0 + t0, nt,
+                                                       strides, ctx->stream);
+                if (e != hipSuccess) return hip_fail("MFMA GEMM launch", e);
+            }
         }
     } else {
         if (quantize)

@@ -416,7 +416,9 @@ bool wide_gemm_supported(const DeviceTensor &t) {
 hipError_t launch_wide_gemm(const DeviceTensor *const *tensors, float *const *outputs, uint32_t count,
                             const uint8_t *image, const float *scales, uint32_t batch, const uint32_t *output_strides,
                             hipStream_t stream, bool accumulate, const float *const *biases, bool swiglu) {
-    if (count == 0 || count > static_cast<uint32_t>(kMaxGroup) || !image || !scales || batch == 0)
+    // a launch holds 65535 token tiles (grid y)
+    if (count == 0 || count > static_cast<uint32_t>(kMaxGroup) || !image || !scales || batch == 0 ||
+        batch > 65535u * 16 * kTokenGroups)
         return hipErrorInvalidValue;
     const DeviceTensor &t0 = *tensors[0];
     for (uint32_t i = 0; i < count; ++i) {

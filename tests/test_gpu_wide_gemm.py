@@ -113,3 +113,29 @@ def test_every_call_adds_its_kernel_time(gpu_ctx):
         gpu_ctx.release(h)
     steps = np.diff(ms)
     assert (steps > 0).all() and steps.max() < 100.0
+
+
+@pytest.mark.parametrize("N,M", [
+    (40, 16384 + 77),        # the images' second span, from its first token on
+    (1, 65535 * 64 + 17),    # more token tiles than one launch holds
+])
+def test_host_batches_of_any_length(hip_lib, N, M):
+    """One call over more tokens than one set of images, every value against
+    the exact product of the codes."""
+    K = 32
+    rng = np.random.default_rng(N)
+    w = synth.q4_0_weights(rng, N, K)
+    block = w.reshape(N, 18)
+    d = block[:, :2].copy().view(np.float16).astype(np.float64)
+    code = np.stack((block[:, 2:] & 15, block[:, 2:] >> 4), axis=-1).reshape(N, K).astype(np.int32) - 8
+    q8 = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    xs = (0.5 + np.arange(M) % 31 / 16.0).astype(np.float32)
+    with abi.Context(hip_lib, device=0) as ctx:   # its buffers go with it
+        h = ctx.upload(w, "q4_0", N, K)
+        y = ctx.gemm(h, q8, N, K, scales=xs)
+        ctx.release(h)
+    for t0 in range(0, M, 1 << 20):
+        q, s = q8[t0:t0 + (1 << 20)], xs[t0:t0 + (1 << 20), None]
+        ref = (q.astype(np.float64) @ code.T.astype(np.float64)) * d.T * s   # one block a row
+        # an fp32 product by the block's scale, one by the token's
+        assert (np.abs(y[t0:t0 + (1 << 20)] - ref) <= 3 * 2.0 ** -24 * np.abs(ref)).all()
