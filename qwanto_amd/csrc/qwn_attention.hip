@@ -942,7 +942,8 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const float *__restri
     if (lane == 0) red_s[1][wave] = total;
     __syncthreads();
     total = (red_s[1][0] + red_s[1][1]) + (red_s[1][2] + red_s[1][3]);
-    const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+    // a NaN sum (a non-finite query or score in any split) is the output's
+    const float inv = total == 0.0f ? 0.0f : 1.0f / total;
     if constexpr (PRE > 0) {
         const uint32_t d = tid % D, part = tid / D;
         float o = 0.0f;

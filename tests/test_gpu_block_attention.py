@@ -75,3 +75,30 @@ def test_tree_matches_oracle_paths(gpu_ctx, oracle_lib, heads, kv_heads, head_di
         env = oracle_envelope(oracle_lib, model, ids, refs, SEEDS)[:, -1:]
         ok, msg = within_envelope(step_errors([rows[i]], refs[-1:]), env)
         assert ok, f"node {i}: {msg}"
+
+
+def run_prefill(gpu_ctx, model, ids, max_ctx):
+    """A long block's logits: its attention in one split (max_ctx 512), or in two and a merge (1500)."""
+    dec = abi.ResidentDecoder(gpu_ctx, dict(model, cfg=dict(model["cfg"], max_ctx=max_ctx)))
+    try:
+        return dec.prefill(ids)[0]
+    finally:
+        dec.close()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_non_finite_queries_show_in_every_split_plan(gpu_ctx, head_dim, bad):
+    """A head whose query is not finite gives NaN, and the other heads their
+    values, whether its context is read in one split or merged from two: the
+    same logits (a merge that drops the NaN leaves a plain zero there)."""
+    rng = np.random.default_rng(head_dim)
+    cfg = dict(config(2, 1, head_dim), layers=1)
+    model = synth.decoder_model(rng, cfg, "q4_0", biases="q")
+    model["layers"][0]["q_bias"][:head_dim] = bad
+    ids = synth.prompt_tokens(rng, cfg["vocab"], 70)
+    one, two = (run_prefill(gpu_ctx, model, ids, n) for n in (512, 1500))
+    model["layers"][0]["q_bias"][:head_dim] = 0.0
+    assert np.linalg.norm(one - run_prefill(gpu_ctx, model, ids, 512)) > 0.1 * np.linalg.norm(one)   # it shows
+    # one int8 step of the other heads' outputs between the two plans' sums
+    assert np.linalg.norm(one - two) <= 1e-2 * np.linalg.norm(one)
