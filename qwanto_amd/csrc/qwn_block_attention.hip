@@ -142,10 +142,12 @@ __global__ __launch_bounds__(64 * kWaves, D <= 128 ? 2 : 1) void block_attention
         for (int g = 0; g < NG; ++g) ks[g] = *reinterpret_cast<const float4 *>(sc + static_cast<size_t>(g) * c.quads * 64);
     };
     auto load_value_group = [&](uint32_t b0, int g) {
-        const uint32_t off = min(b0 / kKvPageTokens + kq, c.pages - 1) * kPage + col * 16;
+        // 64-bit to the block's first page: a head's values pass 2^32 bytes at 16 M tokens of head_dim 256
+        const uint32_t page = b0 / kKvPageTokens;
+        const int8_t *pg = vbase + static_cast<size_t>(page) * kPage;
+        const uint32_t off = min(kq, c.pages - 1 - page) * kPage + col * 16;
 #pragma unroll
-        for (int n = 0; n < 4; ++n)
-            vb[g][n] = *reinterpret_cast<const att_v4i *>(vbase + (off + g * 1024 + n * 256));
+        for (int n = 0; n < 4; ++n) vb[g][n] = *reinterpret_cast<const att_v4i *>(pg + (off + g * 1024 + n * 256));
     };
     auto load_values = [&](uint32_t b0) {
         const float *sc = vsbase + b0 + 4 * col;
