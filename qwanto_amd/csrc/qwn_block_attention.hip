@@ -20,6 +20,7 @@ namespace {
 
 constexpr int kWaves = 4;       // waves per workgroup, each taking every fourth 64-token block
 constexpr int kRows = 16;       // (token, head) rows per workgroup
+constexpr float kTinyMax = 0x1p-100f, kLift = 0x1p80f;   // maxima below are lifted before their split
 constexpr int kPieceRow = 80;   // LDS bytes between the rows of a piece tile: 64 tokens + 16 (bank spread)
 
 struct BlockAttnArgs {
@@ -41,6 +42,7 @@ __device__ __forceinline__ float round_magic(float x, float inv) { return fmaf(x
 // The three int8 pieces of x (scale s1 = amax / 127, inv1 = 1 / s1), each in
 // the low byte of its word: x ~= s1 (p0 + p1 / 254 + p2 / 64516), every
 // residual exact by fma, so no piece passes +-127 and nothing is clamped.
+// amax >= kTinyMax (64516 / s1 stays finite); smaller ones are lifted first.
 __device__ __forceinline__ void split_pieces(float x, float s1, float inv1, uint32_t (&p)[3]) {
     const float y0 = round_magic(x, inv1);
     const float r0 = fmaf(-(y0 - 12582912.0f), s1, x);
@@ -181,20 +183,22 @@ __global__ __launch_bounds__(64 * kWaves, D <= 128 ? 2 : 1) void block_attention
         bad = fmaxf(bad, __shfl_xor(bad, 16));
         bad = fmaxf(bad, __shfl_xor(bad, 32));
         // a maximum below 2^-100 would overflow its reciprocal's multiples:
-        // such a row's scores are 0 to fp32 precision
-        const bool live = amax >= 0x1p-100f && bad == 0.0f;
+        // such a row is split after an exact lift
+        const float lift = amax < kTinyMax ? kLift : 1.0f;
+        amax *= lift;
+        const bool live = amax > 0.0f && bad == 0.0f;
         const float s1 = live ? amax * (1.0f / 127.0f) : 0.0f, inv1 = live ? 127.0f / amax : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t p[4][3];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) split_pieces(live ? f4_at(qv[g][i], e) : 0.0f, s1, inv1, p[e]);
+            for (int e = 0; e < 4; ++e) split_pieces(live ? f4_at(qv[g][i], e) * lift : 0.0f, s1, inv1, p[e]);
 #pragma unroll
             for (int j = 0; j < 3; ++j)
                 qa[j][g][i] = static_cast<int>(pack_low_bytes(p[0][j], p[1][j], p[2][j], p[3][j]));
             __builtin_amdgcn_sched_barrier(0);
         }
-        const float sq = bad > 0.0f ? __builtin_nanf("") : s1;
+        const float sq = bad > 0.0f ? __builtin_nanf("") : lift == 1.0f ? s1 : s1 * (1.0f / kLift);
 #pragma unroll
         for (int r = 0; r < 4; ++r) qs[g][r] = __shfl(sq, 4 * kq + r);
     }
@@ -270,23 +274,41 @@ __global__ __launch_bounds__(64 * kWaves, D <= 128 ? 2 : 1) void block_attention
                 sum += p[i];
             }
             l_run[r] = fmaf(l_run[r], alpha[r], row16_sum(sum));
+            float pv[NG][NT], am[NG];
+            uint32_t least = 0xffffffffu;   // of the maxima above 0, as bits less one
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
-                float pv[NT], am = 0.0f;
+                am[g] = 0.0f;
 #pragma unroll
                 for (int i = 0; i < NT; ++i) {
                     // masked tokens' scales may be any bits
-                    pv[i] = p[i] == 0.0f ? 0.0f : p[i] * f4_at(vs[g], i);
-                    am = fmaxf(am, pv[i]);
+                    pv[g][i] = p[i] == 0.0f ? 0.0f : p[i] * f4_at(vs[g], i);
+                    am[g] = fmaxf(am[g], pv[g][i]);
                 }
-                am = row16_max(am);
-                const bool live = am >= 0x1p-100f;
-                const float s1 = live ? am * (1.0f / 127.0f) : 0.0f, inv1 = live ? 127.0f / am : 0.0f;
-                ps1[g][r] = s1;
+                am[g] = row16_max(am[g]);
+                least = min(least, __builtin_bit_cast(uint32_t, am[g]) - 1u);
+                ps1[g][r] = 1.0f / 127.0f;
+            }
+            // rare (a block far below its row's maximum, or values that
+            // small): one test for the wave
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(least < __builtin_bit_cast(uint32_t, kTinyMax) - 1u) != 0, 0)) {
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    const float lift = am[g] < kTinyMax ? kLift : 1.0f;
+                    ps1[g][r] *= 1.0f / lift;
+                    am[g] *= lift;
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) pv[g][i] *= lift;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const float s1 = am[g] * (1.0f / 127.0f), inv1 = am[g] > 0.0f ? 127.0f / am[g] : 0.0f;
+                ps1[g][r] *= am[g];
 #pragma unroll
                 for (int i = 0; i < NT; ++i) {
                     uint32_t q[3];
-                    split_pieces(pv[i], s1, inv1, q);
+                    split_pieces(pv[g][i], s1, inv1, q);
                     uint8_t *dst = pp + (g * 3 * kRows + 4 * kq + r) * kPieceRow + 16 * i + col;
 #pragma unroll
                     for (int j = 0; j < 3; ++j) dst[j * kRows * kPieceRow] = static_cast<uint8_t>(q[j]);

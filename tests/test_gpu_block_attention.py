@@ -102,3 +102,41 @@ def test_non_finite_queries_show_in_every_split_plan(gpu_ctx, head_dim, bad):
     assert np.linalg.norm(one - run_prefill(gpu_ctx, model, ids, 512)) > 0.1 * np.linalg.norm(one)   # it shows
     # one int8 step of the other heads' outputs between the two plans' sums
     assert np.linalg.norm(one - two) <= 1e-2 * np.linalg.norm(one)
+
+
+@pytest.mark.parametrize("max_ctx", [512, 1500])
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_tiny_queries_choose(gpu_ctx, oracle_lib, head_dim, max_ctx):
+    """Queries of 2^-103 against keys of 2^105: scores that choose among the tokens."""
+    rng = np.random.default_rng(head_dim + 1)
+    cfg = dict(config(2, 1, head_dim), layers=1, max_ctx=max_ctx)
+    model = synth.decoder_model(rng, cfg, "q4_0", biases="qk")
+    layer = model["layers"][0]
+    for p, scale in (("q", 2.0 ** -103), ("k", 2.0 ** 105)):
+        layer[p].reshape(-1, 18)[:, :2] = 0   # the projection is its bias
+        layer[p + "_bias"] *= np.float32(scale)
+    ids = synth.prompt_tokens(rng, cfg["vocab"], 70)
+    ref = oracle_lib.decoder(model)
+    refs = [ref.forward(int(t)) for t in ids]
+    ref.close()
+    env = oracle_envelope(oracle_lib, model, ids, refs, SEEDS)[:, -1:]
+    ok, msg = within_envelope(step_errors([run_prefill(gpu_ctx, model, ids, max_ctx)], refs[-1:]), env)
+    assert ok, msg
+
+
+@pytest.mark.parametrize("max_ctx", [512, 1500])
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_tiny_values_come_through(gpu_ctx, oracle_lib, head_dim, max_ctx):
+    """Values of 2^-95 and an all-zero embedding row, so the attention is all there is of the logits."""
+    rng = np.random.default_rng(head_dim + 2)
+    cfg = dict(config(2, 1, head_dim), layers=1, max_ctx=max_ctx)
+    model = synth.decoder_model(rng, cfg, "q4_0", biases="qkv")
+    model["layers"][0]["v_bias"] *= np.float32(2.0 ** -95)
+    model["embed"][0] = 0
+    ids = np.zeros(70, dtype=np.int32)
+    ref = oracle_lib.decoder(model)
+    want = [ref.forward(0) for _ in ids][-1].astype(np.float64)
+    ref.close()
+    got = run_prefill(gpu_ctx, model, ids, max_ctx)
+    # one step of the int8 input of o at the most: 1/127 of the largest value
+    assert np.linalg.norm(want) > 0 and np.linalg.norm(got - want) <= 1e-2 * np.linalg.norm(want)
