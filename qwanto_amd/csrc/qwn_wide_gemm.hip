@@ -6,9 +6,10 @@
 // workgroup of its own, so every sixteen tokens load and decode the weights
 // again and fetch their own activations: 64 tokens through one Qwen2-1.5B
 // Q4_0 layer take 34 us of GEMMs, 1003 tokens 545 us in sixteen such blocks.
-// Here a workgroup takes 64 or 128 rows x 64 tokens, its activations staged
-// through LDS once for its four waves: the 1003 tokens take 201 us in four
-// launches, and the whole prompt through two layers 0.68 ms instead of 2.57.
+// Here a workgroup takes 64 or 128 rows x 64 tokens (fewer tokens where that
+// leaves CUs without one), its activations staged through LDS once for its
+// four waves: the 1003 tokens take 201 us in four launches, and the whole
+// prompt through two layers 0.62 ms instead of 2.57.
 // The gate/up launch (55 GFLOP, 97 us, 0.57 PFLOP/s) keeps the vector ALU
 // busy half of the time and the matrix cores a quarter: waits for a unit's
 // loads and the last, half-filled round of workgroups take the rest.
@@ -39,7 +40,7 @@ typedef _Float16 wide_v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 wide_v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kWideWaves = 4;           // waves of a set: 16 RT rows each
-constexpr int kTokenGroups = 4;         // 16-token groups of a workgroup
+constexpr int kTokenGroups = 4;         // 16-token groups of a workgroup (two where few tiles exist)
 constexpr uint32_t kUnitImage = 4096;   // image bytes of one unit of a 16-token group (without the sums)
 
 struct WideArgs {
@@ -353,7 +354,8 @@ __global__ __launch_bounds__(64 * kWideWaves * KW, KW < 4 ? 2 : 4) void wide_gem
 }
 
 struct WidePlan {
-    uint32_t rt = 0, kw = 1;   // row groups per wave, sets of waves splitting K
+    uint32_t rt = 0, kw = 1;      // row groups per wave, sets of waves splitting K
+    uint32_t tt = kTokenGroups;   // 16-token groups per workgroup
 };
 
 template <int KIND, int RT, int TT, int KW, bool PAIR>
@@ -373,7 +375,10 @@ hipError_t launch_wide_kind(const WideArgs &a, const WidePlan &p, bool pair, dim
     switch (p.kw) {
     case 1: return launch_wide_one<KIND, 1, kTokenGroups, 1, false>(a, grid, stream);
     case 2: return launch_wide_one<KIND, 1, kTokenGroups, 2, false>(a, grid, stream);
-    default: return launch_wide_one<KIND, 1, kTokenGroups, 4, false>(a, grid, stream);
+    default:
+        if (p.tt == 1) return launch_wide_one<KIND, 1, 1, 4, false>(a, grid, stream);
+        if (p.tt == 2) return launch_wide_one<KIND, 1, 2, 4, false>(a, grid, stream);
+        return launch_wide_one<KIND, 1, kTokenGroups, 4, false>(a, grid, stream);
     }
 }
 
@@ -384,6 +389,12 @@ hipError_t launch_wide_kind(const WideArgs &a, const WidePlan &p, bool pair, dim
 // 1x2 67, 1x4 77; 333 x 2560 x 9728 HyperVSQ-2: 47, 41, 38, 31, 30 (four K
 // splits added with float atomics: 55 and 37).  128-token tiles: 131 and 78,
 // and no faster for the pairs (1003 tokens x 2 x 8960 x 1536: 99 against 97).
+// Four sets in a half (a quarter) of the CUs or fewer: each unit is a round of
+// vector instructions of all its waves, so tiles of 32 (16) tokens on twice
+// (four times) the workgroups.  65 tokens x 1536 x 8960 Q4_0 as a host call's
+// kernels, 64-, 32-, 16-token tiles: 38.6, 30.1, 26.0 us; 65 x 2560 x 9728:
+// 41.2 and 31.4; a 65-token prompt of the 1.5B-shaped decoder 3.40, 2.94 and
+// 2.71 ms (3.17 as a narrow block of 64 and one of 1).
 WidePlan wide_plan(const DeviceTensor *const *tensors, uint32_t count, uint32_t batch, bool pair) {
     const uint32_t token_tiles = (batch + 16 * kTokenGroups - 1) / (16 * kTokenGroups);
     auto tiles = [&](uint32_t rt) {
@@ -399,6 +410,7 @@ WidePlan wide_plan(const DeviceTensor *const *tensors, uint32_t count, uint32_t 
     p.rt = 1;
     const uint32_t sets = tiles(1) <= kChipCus ? 4 : tiles(1) < 4 * kChipCus ? 2 : 1;
     while (p.kw < sets && tensors[0]->units >= 4 * p.kw) p.kw *= 2;
+    if (p.kw == 4 && 2 * tiles(1) <= kChipCus) p.tt = 4 * tiles(1) <= kChipCus ? 1 : 2;
     return p;
 }
 
@@ -451,7 +463,7 @@ hipError_t launch_wide_gemm(const DeviceTensor *const *tensors, float *const *ou
     a.scales = scales;
     a.ntok = batch;
     a.accumulate = accumulate ? 1u : 0u;
-    const dim3 dims(grid, (batch + 16 * kTokenGroups - 1) / (16 * kTokenGroups));
+    const dim3 dims(grid, (batch + 16 * p.tt - 1) / (16 * p.tt));
     return t0.kind == kHvsq2 ? launch_wide_kind<kHvsq2>(a, p, swiglu, dims, stream)
                              : launch_wide_kind<kQ4_0>(a, p, swiglu, dims, stream);
 }

@@ -59,6 +59,8 @@ def test_wide_prefill_matches_oracle(gpu_ctx, oracle_lib, dtype, shape, prompt, 
     (2560, 1536, 160),   # two sets
     (9000, 520, 129),    # one set
     (17000, 256, 300),   # two row groups a wave, fewer units than sets
+    (100, 2000, 81),     # 16-token tiles, the last of one token
+    (2240, 2000, 161),   # 32-token tiles, the last of one token
 ])
 def test_host_batches(gpu_ctx, oracle_lib, dtype, N, K, M):
     """qwn_cuda_abi_hypervsq2_gemm with more than 16 tokens."""
