@@ -768,7 +768,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *handle, const 
         part(reinterpret_cast<void **>(&d->pv), P * KV * 4);
         part(reinterpret_cast<void **>(&d->pattn), P * Q * 4);
         part(reinterpret_cast<void **>(&d->pgate), P * I * 4);
-        part(reinterpret_cast<void **>(&d->pup), P * I * 4);
+        // a wide block's gate/up are stored as one, silu(gate) * up: pup is a narrow block's
+        part(reinterpret_cast<void **>(&d->pup), kBlockTokens * I * 4);
         part(reinterpret_cast<void **>(&d->pscales), P * 4);
         part(reinterpret_cast<void **>(&d->ppos), P * 4);
         size_t stride = 0;

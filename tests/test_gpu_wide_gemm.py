@@ -141,3 +141,21 @@ def test_host_batches_of_any_length(hip_lib, N, M):
         ref = (q.astype(np.float64) @ code.T.astype(np.float64)) * d.T * s   # one block a row
         # an fp32 product by the block's scale, one by the token's
         assert (np.abs(y[t0:t0 + (1 << 20)] - ref) <= 3 * 2.0 ** -24 * np.abs(ref)).all()
+
+
+def test_wide_decoder_memory(gpu_ctx):
+    """A decoder holds one [1024][intermediate] activation for its long
+    blocks (gate/up are stored as one), not two."""
+    import torch
+    cfg = config(256, 16384, 2, 1, 128, 1024)
+    model = synth.decoder_model(np.random.default_rng(3), cfg, "q4_0")
+    free = torch.cuda.mem_get_info()[0]
+    dec = abi.ResidentDecoder(gpu_ctx, model)
+    try:
+        used = free - torch.cuda.mem_get_info()[0]
+        assert dec.prefill(synth.prompt_tokens(np.random.default_rng(4), 500, 1024))[0].shape == (500,)
+    finally:
+        dec.close()
+    act = 1024 * 16384 * 4
+    # the activation, its f16 image (half), and about 16 MB of weights with their MFMA-order copies
+    assert act < used < act + act // 2 + (40 << 20), used
