@@ -1021,8 +1021,6 @@ struct MfmaAttnArgs {
     float scale;
     uint32_t position;
     const int32_t *position_ptr;
-    const uint64_t *tree_mask;  // optional: the query token's ancestor mask over slots *tree_base + a
-    const int32_t *tree_base;
 };
 
 __device__ __forceinline__ int piece_round(float v) {
@@ -1099,8 +1097,6 @@ __global__ __launch_bounds__(64 * NW) void mfma_attention_kernel(MfmaAttnArgs a)
     }
     const uint32_t t1 = min(tokens, t0 + a.split);
     const uint32_t col = lane % 16, kq = lane / 16;   // MFMA column / k-quarter of this lane
-    const uint64_t tmask = a.tree_mask ? *a.tree_mask : 0ull;
-    const uint32_t tbase = a.tree_mask ? static_cast<uint32_t>(*a.tree_base) : 0xffffffffu;
 
     // 1. query pieces (A of the scores), this lane: head (col / 4) of row
     //    tile rt, piece col % 4, channels 64g + 16kq .. +15.  Where the
@@ -1241,7 +1237,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_attention_kernel(MfmaAttnArgs a)
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
             const uint32_t t = b0 + 16 * i + col;
-            valid[i] = t < t1 && tree_attends(t, tbase, tmask);
+            valid[i] = t < t1;
         }
 
 #pragma unroll
@@ -1519,14 +1515,9 @@ hipError_t launch_attention_merge(const float *partials, float *output, uint32_t
 
 hipError_t launch_mfma_attention(const KvCache &c, const float *query, float *output, float *partials,
                                  uint32_t query_heads, uint32_t position, const int32_t *position_ptr,
-                                 uint32_t span, float scale, hipStream_t stream, const uint64_t *tree_mask,
-                                 const int32_t *tree_base) {
-    if (!mfma_attention_supported(c, query_heads) || span == 0 || span > c.max_tokens ||
-        (!tree_mask) != (!tree_base))
-        return hipErrorInvalidValue;
+                                 uint32_t span, float scale, hipStream_t stream) {
+    if (!mfma_attention_supported(c, query_heads) || span == 0 || span > c.max_tokens) return hipErrorInvalidValue;
     MfmaAttnArgs args{};
-    args.tree_mask = tree_mask;
-    args.tree_base = tree_base;
     args.c = c;
     args.query = query;
     args.output = output;
@@ -1670,13 +1661,11 @@ size_t attention_at_workspace_floats(const KvCache &c, uint32_t query_heads) {
 }
 
 hipError_t launch_attention_at(const KvCache &c, const float *query, float *output, uint32_t query_heads,
-                               const int32_t *position_ptr, float scale, float *partials, hipStream_t stream,
-                               const uint64_t *tree_mask, const int32_t *tree_base) {
+                               const int32_t *position_ptr, float scale, float *partials, hipStream_t stream) {
     if (query_heads == 0 || c.head_dim > 1024) return hipErrorInvalidValue;
     if (mfma_attention_supported(c, query_heads))
         return launch_mfma_attention(c, query, output, partials, query_heads, 0, position_ptr, c.max_tokens, scale,
-                                     stream, tree_mask, tree_base);
-    if (tree_mask) return hipErrorInvalidValue;  // tree masks: the MFMA and decode kernels only
+                                     stream);
     AttnArgs args{};
     args.c = c;
     args.query = query;

@@ -421,11 +421,11 @@ hipError_t enqueue_prefill(Decoder *d, uint32_t m, uint32_t kind, hipStream_t s,
             }
             if ((e = launch_decode_attention(at, s)) != hipSuccess) return e;
         } else {
+            // other head shapes, one token at a time (never a tree's block: verify_tree refuses them)
             for (uint32_t i = 0; i < m; ++i)
                 if ((e = launch_attention_at(d->caches[l], d->pq + static_cast<size_t>(i) * Q,
                                              d->pattn + static_cast<size_t>(i) * Q, d->heads, d->ppos + i,
-                                             d->attn_scale, d->partials, s, tree ? d->tree_mask + row0 + i : nullptr,
-                                             tree ? d->tree_base : nullptr)) != hipSuccess)
+                                             d->attn_scale, d->partials, s)) != hipSuccess)
                     return e;
         }
         // on the MFMA path with the MFMA-order copy the gate/up launch stores
@@ -1161,7 +1161,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_verify_tree(QwnCudaContextHandle *handle, Q
         mask[i] = (p < 0 ? 0ull : mask[p]) | (1ull << i);
         pos[i] = static_cast<int32_t>(d->position + depth[i]);
     }
-    // the masked attention runs in the one-split decode kernel or the MFMA kernel
+    // the masked attention runs in the one-split decode kernel or the block
+    // kernel, for up to eight query heads per KV head
     if (!d->fused_attention && !mfma_attention_supported(d->caches[0], d->heads)) {
         set_error("tree verify needs the decode or MFMA attention for this head shape");
         return QWN_CUDA_STATUS_UNSUPPORTED;

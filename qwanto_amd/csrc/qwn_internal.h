@@ -409,8 +409,7 @@ size_t mfma_attention_workspace_floats(const KvCache &c, uint32_t query_heads, u
 uint32_t mfma_attention_launches(const KvCache &c, uint32_t query_heads, uint32_t span);
 hipError_t launch_mfma_attention(const KvCache &c, const float *query, float *output, float *partials,
                                  uint32_t query_heads, uint32_t position, const int32_t *position_ptr,
-                                 uint32_t span, float scale, hipStream_t stream,
-                                 const uint64_t *tree_mask = nullptr, const int32_t *tree_base = nullptr);
+                                 uint32_t span, float scale, hipStream_t stream);
 bool decode_attention_supported(const KvCache &c, uint32_t query_heads);
 uint32_t decode_split_tokens(const KvCache &c, uint32_t tokens);
 size_t decode_attention_workspace_floats(const KvCache &c, uint32_t query_heads, uint32_t tokens);
@@ -452,12 +451,9 @@ constexpr uint32_t kDevicePositionSplit = 64;
 hipError_t launch_kv_append_at(const KvCache &c, const float *key, const float *value,
                                const int32_t *token_ptr, hipStream_t stream);
 size_t attention_at_workspace_floats(const KvCache &c, uint32_t query_heads);
-// tree_mask / tree_base: a draft-tree node's ancestor mask (as in
-// DecodeAttentionLaunch; needs the MFMA attention, mfma_attention_supported).
 hipError_t launch_attention_at(const KvCache &c, const float *query, float *output,
                                uint32_t query_heads, const int32_t *position_ptr, float scale,
-                               float *partials, hipStream_t stream, const uint64_t *tree_mask = nullptr,
-                               const int32_t *tree_base = nullptr);
+                               float *partials, hipStream_t stream);
 
 // Keeps a draft tree's accepted path: for k < len, the K/V and scales of
 // slot base + path[k] move to slot base + k (path strictly increasing from
