@@ -1,14 +1,15 @@
-"""Prompts of more than one narrow block: the projections on the wide GEMM
-(qwn_wide_gemm.hip), through the resident decoder, against the oracle.  Token
-counts that end inside a 16-token group and a token tile, rows that end
-inside a row tile and a 16-row group, K that ends inside a unit, the K split
-of the residual adds, gate/up pairs, biases, a prompt of more than one wide
-block.  The logits of the last token are held to the oracle's rounding
-envelope (parity.py)."""
+"""More than one narrow block of tokens on the wide GEMM (qwn_wide_gemm.hip):
+prompts through the resident decoder and host batches, against the oracle.
+Token counts that end inside a 16-token group and a token tile, rows that end
+inside a row tile and a 16-row group, K that ends inside a unit, every tile
+and K split of the plan, gate/up pairs, biases, prompts of more than one wide
+block.  A prompt's logits are held to the oracle's rounding envelope
+(parity.py).  Then the host batch around it: results in pieces, long batches,
+telemetry."""
 import numpy as np
 import pytest
 
-from parity import oracle_envelope, step_errors, within_envelope
+from parity import gemv_close, oracle_envelope, step_errors, within_envelope
 from qwanto_amd import abi, synth
 from test_gpu_gemv import check_hvsq2, check_q4_0
 
@@ -27,8 +28,10 @@ def config(hidden, inter, heads, kv_heads, head_dim, max_ctx):
     ((256, 512, 2, 1, 128, 512), 65, False),       # one token past the narrow block
     ((288, 1056, 3, 1, 64, 512), 129, True),  # rows and K ending inside every tile and unit
     ((544, 2336, 2, 2, 128, 1200), 300, False),
-    ((256, 9728, 2, 1, 64, 1200), 520, False),     # 8-group token tiles of the gate/up pair, the K split of down
-    ((256, 256, 1, 1, 64, 1200), 1100, True),      # a wide block and a second, narrow one's remainder
+    ((256, 9728, 2, 1, 64, 1200), 520, False),     # the K split of down, four ways
+    ((256, 256, 1, 1, 64, 1200), 1100, True),      # a wide block and a second one of 76 tokens
+    ((256, 256, 1, 1, 64, 1200), 1025, False),     # from a wide block, launched as it is, to a captured one of one token
+    ((256, 256, 2, 1, 64, 1200), 1050, True),      # ... and of 26
 ])
 def test_wide_prefill_matches_oracle(gpu_ctx, oracle_lib, dtype, shape, prompt, bias):
     rng = np.random.default_rng(shape[1] + prompt)
@@ -54,13 +57,16 @@ def test_wide_prefill_matches_oracle(gpu_ctx, oracle_lib, dtype, shape, prompt, 
 @pytest.mark.parametrize("dtype", ["q4_0", "hvsq2"])
 @pytest.mark.parametrize("N,K,M", [
     (1, 31, 65),         # one row, K inside one unit, a one-token last group
-    (77, 777, 70),       # rows and K ending inside their tiles; four sets of waves splitting K
+    # by wide_plan on 256 CUs: 16-row groups a wave x sets of waves splitting K, tokens of a tile
+    (77, 777, 70),       # rows and K ending inside their tiles; 1 x 2, 64
     (130, 129, 40),      # 17 to 64 tokens: several groups on the 16-token GEMM
-    (2560, 1536, 160),   # two sets
-    (9000, 520, 129),    # one set
-    (17000, 256, 300),   # two row groups a wave, fewer units than sets
-    (100, 2000, 81),     # 16-token tiles, the last of one token
-    (2240, 2000, 161),   # 32-token tiles, the last of one token
+    (2560, 1536, 160),   # Q4_0 1 x 4, 32; HyperVSQ-2 1 x 2, 64
+    (9000, 520, 129),    # Q4_0 1 x 2, HyperVSQ-2 1 x 1, 64
+    (17000, 256, 300),   # 1 x 1, 64: more workgroups than CUs, one or two units
+    (100, 2000, 81),     # 1 x 4, 16, the last tile of one token
+    (2240, 2000, 161),   # 1 x 4, 32, the last tile of one token
+    (2500, 2000, 257),   # 1 x 4, 64, the last tile of one token, sets of unequal length
+    (9700, 600, 833),    # 2 x 1, 64: several units, the last ones part filled
 ])
 def test_host_batches(gpu_ctx, oracle_lib, dtype, N, K, M):
     """qwn_cuda_abi_hypervsq2_gemm with more than 16 tokens."""
@@ -68,22 +74,46 @@ def test_host_batches(gpu_ctx, oracle_lib, dtype, N, K, M):
     check(gpu_ctx, oracle_lib, N, K, seed=N + K + M, M=M)
 
 
+@pytest.mark.parametrize("dtype", ["q4_0", "hvsq2"])
+@pytest.mark.parametrize("N,K,M", [(77, 300, 40), (130, 520, 100), (1030, 777, 129)])
+def test_host_batches_of_fp32_tokens(gpu_ctx, oracle_lib, dtype, N, K, M):
+    """fp32 tokens, quantized on the device behind the images of several
+    groups: the oracle's product of its own quantized tokens."""
+    rng = np.random.default_rng(N + M)
+    w, x = synth.weights(dtype, rng, N, K), synth.activations(rng, M, K)
+    q8, xs, sums = oracle_lib.quantize(x)
+    h = gpu_ctx.upload(w, dtype, N, K)
+    try:
+        y = gpu_ctx.gemm(h, x, N, K)
+    finally:
+        gpu_ctx.release(h)
+    for t in range(M):
+        ref = (oracle_lib.gemv_q4_0_q8(w, q8[t], float(xs[t]), K, N) if dtype == "q4_0" else
+               oracle_lib.gemv_hvsq2(w, q8[t], sums[t], float(xs[t]), K, N))
+        ok, worst = gemv_close(y[t], ref)
+        assert ok, f"token {t}: worst {worst:.3g} of tolerance"
+
+
 @pytest.mark.parametrize("N,M", [
-    (65537, 1),      # one token past the rows that are stored to the host directly: a ragged last piece
+    (65537, 1),      # one row past those that are stored to the host directly: a ragged last piece
     (1021, 150),     # rows that pieces end inside of
     (70003, 300),    # many windows
 ])
 def test_host_results_in_pieces(gpu_ctx, oracle_lib, N, M):
     """Results as the device wrote them, piece by piece, into rows of a larger
-    stride: every value there, the gaps untouched, twice over."""
+    stride: every value there, the gaps untouched.  Every row of every pass
+    has a scale of its own, so a piece that another row, window or pass left
+    behind is another value."""
     import ctypes
     rng = np.random.default_rng(N + M)
     w = synth.q4_0_weights(rng, N, 64)
-    q8 = rng.integers(-127, 128, (M, 64), dtype=np.int8)
-    xs = np.linspace(0.5, 1.5, M, dtype=np.float32)
+    token = rng.integers(-127, 128, 64, dtype=np.int8)
+    q8 = np.tile(token, (M, 1))
+    ref = oracle_lib.gemv_q4_0_q8(w, token, 1.0, 64, N)
     h = gpu_ctx.upload(w, "q4_0", N, 64)
     try:
-        for _ in range(2):
+        for turn in range(3):
+            xs = (1.0 + np.arange(M) / 256.0 + 4.0 * turn).astype(np.float32)
             out = np.full((M, N + 3), np.nan, dtype=np.float32)
             req = abi.GemmRequest(tensor=h, input_q8=q8.ctypes.data, input_scale=0.0, input_scales=xs.ctypes.data,
                                   output=out.ctypes.data, batch=M, rows=N, cols=64, input_stride=64,
@@ -92,10 +122,9 @@ def test_host_results_in_pieces(gpu_ctx, oracle_lib, N, M):
             gpu_ctx.lib.check("gemm", gpu_ctx.lib.lib.qwn_cuda_abi_hypervsq2_gemm(gpu_ctx._h, ctypes.byref(req),
                                                                                 ctypes.byref(tm)))
             assert np.isnan(out[:, N:]).all()
-            for t in sorted({0, M // 2, M - 1}):
-                ref = oracle_lib.gemv_q4_0_q8(w, q8[t], float(xs[t]), 64, N)
-                assert np.allclose(out[t, :N], ref, rtol=1e-5, atol=1e-5 * np.abs(ref).max())  # two fp32 sums of two products
-            assert not np.isnan(out[:, :N]).any()
+            # two fp32 sums of two products; neighbouring scales are 2^-11 or more apart
+            want = ref[None, :] * xs[:, None]
+            assert np.allclose(out[:, :N], want, rtol=1e-5, atol=1e-5 * np.abs(ref).max())
     finally:
         gpu_ctx.release(h)
 
