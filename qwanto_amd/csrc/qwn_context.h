@@ -88,6 +88,7 @@ struct DownloadPipe {
     PinnedBuffer data;
     DeviceBuffer counters;  // [2][kDownloadPieces] workgroups done
     uint32_t epoch = 0;
+    double copy_ms = 0.0;   // of the last result: the host's copies out of the windows
 };
 
 struct Context {

@@ -161,6 +161,7 @@ hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const floa
     };
     if ((e = issue(0)) != hipSuccess || (windows > 1 && (e = issue(1)) != hipSuccess)) return e;
     size_t touched = 0;
+    d.copy_ms = 0.0;
     for (size_t w = 0; w < windows; ++w) {
         const uint32_t half = w & 1, np = pieces(w);
         for (uint32_t p = 0; p < np; ++p) {
@@ -192,11 +193,13 @@ hipError_t download_rows(Context *ctx, float *dst, size_t dst_stride, const floa
                 d.counters.release();
                 return failed;
             }
+            const auto t_copy = std::chrono::steady_clock::now();
             for (size_t at = first, end = std::min(total, first + kDownloadPiece); at < end;) {
                 const size_t row = at / cols, col = at % cols, n = std::min(cols - col, end - at);
                 std::memcpy(dst + row * dst_stride + col, pinned + half * kWindow + (at - w * kWindow), n * sizeof(float));
                 at += n;
             }
+            d.copy_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_copy).count();
         }
         // the window is copied out: its memory takes the one after next
         if (w + 2 < windows && (e = issue(w + 2)) != hipSuccess) return e;
@@ -290,7 +293,8 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     // buffer, and the GEMV epilogue stores into the pinned output buffer, so a
     // call is two kernels and one synchronisation instead of three DMA
     // transfers around them.  Outputs of 64K+ rows (the LM head) and the MFMA
-    // path keep the device buffers and DMA.
+    // path take their activations by DMA into a device buffer and leave
+    // through download_rows.
     const bool zero_copy = !mfma && r->rows < 65536;
     if ((e = ctx->host_in.ensure(in_bytes + scale_bytes)) != hipSuccess ||
         (e = ctx->host_out.ensure(zero_copy ? out_bytes : 0)) != hipSuccess ||
@@ -337,6 +341,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
     const size_t mfma_img = (static_cast<size_t>(std::min(r->batch, kImageTokens)) + 15) / 16 * group_img;
     if (mfma && ((e = ctx->dev_work.ensure(mfma_img + (quantize ? in_bytes / 4 : 0))) != hipSuccess))
         return hip_fail("MFMA workspace allocation", e, QWN_CUDA_STATUS_OUT_OF_MEMORY);
+    uint64_t launches = 0;
     (void)hipEventRecord(ctx->ev_start, ctx->stream);
     if (mfma) {
         // int8 tokens on the device: as given, or quantized from fp32 per token
@@ -347,6 +352,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
                                            nullptr, 0, static_cast<float *>(ctx->dev_scales.ptr), dq, dev_stride,
                                            ctx->stream);
             if (e != hipSuccess) return hip_fail("activation quantize launch", e);
+            ++launches;
             q8 = dq;
         }
         uint8_t *img = static_cast<uint8_t *>(ctx->dev_work.ptr);
@@ -360,6 +366,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
             if ((e = qwn::launch_mfma_image(t, q8 + static_cast<size_t>(i0) * dev_stride, ni, dev_stride, img,
                                             ctx->stream, wide)) != hipSuccess)
                 return hip_fail("MFMA image launch", e);
+            ++launches;
             for (uint32_t t0 = 0; t0 < ni; t0 += step) {
                 const uint32_t nt = std::min(step, ni - t0);
                 float *outs[1] = {dev_out + static_cast<size_t>(i0 + t0) * r->rows};
@@ -367,6 +374,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
                          : qwn::launch_gemm_mfma_group(ts, outs, 1, img + (t0 / 16) * group_img, sc + i0 + t0, nt,
                                                        strides, ctx->stream);
                 if (e != hipSuccess) return hip_fail("MFMA GEMM launch", e);
+                ++launches;
             }
         }
     } else {
@@ -379,6 +387,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
                                   ctx->stream);
         if (e != hipSuccess) return hip_fail("activation image launch", e);
         if ((e = qwn::launch_gemv(g, ctx->stream)) != hipSuccess) return hip_fail("GEMV launch", e);
+        launches = 1 + (r->batch + qwn::kMaxTokensPerLaunch - 1) / qwn::kMaxTokensPerLaunch;
     }
     (void)hipEventRecord(ctx->ev_end, ctx->stream);
     const auto t_sync = std::chrono::steady_clock::now();
@@ -386,7 +395,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
                                               r->rows, r->batch)) != hipSuccess)
         return hip_fail("result download", e);
     if (zero_copy && (e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return hip_fail("GEMV synchronize", e);
-    const double sync_ms = ms_since(t_sync);
+    const double sync_ms = ms_since(t_sync) - (zero_copy ? 0.0 : ctx->download.copy_ms);
     if (zero_copy) {
         const float *hout = static_cast<const float *>(ctx->host_out.ptr);
         for (uint32_t b = 0; b < r->batch; ++b)
@@ -404,7 +413,7 @@ int execute_gemm(Context *ctx, const QwnCudaGemmRequest *r, QwnCudaTelemetry *te
 
     QwnCudaTelemetry &tm = ctx->telemetry;
     tm.gpu_matmul_count++;
-    tm.gpu_kernel_launch_count += 1 + (r->batch + qwn::kMaxTokensPerLaunch - 1) / qwn::kMaxTokensPerLaunch;
+    tm.gpu_kernel_launch_count += launches;
     tm.gpu_projection_count++;
     tm.gpu_kernel_ms += kernel_ms;
     tm.gpu_transfer_ms += transfer_ms;

@@ -188,3 +188,18 @@ def test_wide_decoder_memory(gpu_ctx):
     act = 1024 * 16384 * 4
     # the activation, its f16 image (half), and about 16 MB of weights with their MFMA-order copies
     assert act < used < act + act // 2 + (40 << 20), used
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("M,launches", [(1, 2), (16, 2), (64, 2), (65, 2), (16384 + 65, 4)])
+def test_launches_of_a_host_batch(hip_lib, M, launches, f32):
+    """gpu_kernel_launch_count: the images' launches and the GEMMs', and the
+    quantize in front of the MFMA path's for fp32 tokens (the GEMV's image
+    launch quantizes by itself)."""
+    rng = np.random.default_rng(M)
+    x = synth.activations(rng, M, 256) if f32 else rng.integers(-127, 128, (M, 256), dtype=np.int8)
+    with abi.Context(hip_lib, device=0) as ctx:
+        h = ctx.upload(synth.q4_0_weights(rng, 64, 256), "q4_0", 64, 256)
+        n = ctx.telemetry().gpu_kernel_launch_count
+        ctx.gemm(h, x, 64, 256, scales=None if f32 else np.ones(M, dtype=np.float32))
+        assert ctx.telemetry().gpu_kernel_launch_count - n == launches + (f32 and M > 1)
