@@ -82,7 +82,7 @@ typedef struct {
     double decode_ms;             /* wall clock, generated steps */
     uint64_t weight_bytes_per_step; /* algorithmic weight bytes one step reads */
     uint32_t graph;               /* 1 if steps replay a captured HIP graph */
-    uint32_t prefill_block_tokens; /* prompt tokens per prefill block */
+    uint32_t prefill_block_tokens; /* prompt tokens a prefill block of this prompt holds at most */
 } QwnHipDecoderStats;
 
 QWN_CUDA_ABI_API int qwn_hip_decoder_create(QwnCudaContextHandle *context, const QwnHipDecoderDesc *desc,

@@ -1286,7 +1286,8 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_generate(QwnCudaContextHandle *handle, QwnH
         stats->decode_ms = std::chrono::duration<double, std::milli>(t2 - t1).count();
         stats->weight_bytes_per_step = d->weight_bytes;
         stats->graph = d->exec ? 1u : 0u;
-        stats->prefill_block_tokens = d->block_tokens;
+        stats->prefill_block_tokens =
+            prompt_count > d->block_tokens ? std::max(d->wide_tokens, d->block_tokens) : d->block_tokens;
     }
     return QWN_CUDA_STATUS_OK;
 }

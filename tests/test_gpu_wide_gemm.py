@@ -172,6 +172,17 @@ def test_host_batches_of_any_length(hip_lib, N, M):
         assert (np.abs(y[t0:t0 + (1 << 20)] - ref) <= 3 * 2.0 ** -24 * np.abs(ref)).all()
 
 
+@pytest.mark.parametrize("max_ctx,prompt,tokens", [(512, 64, 64), (512, 65, 512), (2048, 300, 1024), (64, 33, 64)])
+def test_block_size_of_a_prompt(gpu_ctx, max_ctx, prompt, tokens):
+    """generate's prefill_block_tokens: narrow blocks up to 64 tokens, else the decoder's wide ones."""
+    rng = np.random.default_rng(max_ctx)
+    dec = abi.ResidentDecoder(gpu_ctx, synth.decoder_model(rng, config(256, 256, 1, 1, 64, max_ctx), "q4_0"))
+    try:
+        assert dec.generate(synth.prompt_tokens(rng, 500, prompt), 1)[1].prefill_block_tokens == tokens
+    finally:
+        dec.close()
+
+
 def test_wide_decoder_memory(gpu_ctx):
     """A decoder holds one [1024][intermediate] activation for its long
     blocks (gate/up are stored as one), not two."""
