@@ -32,9 +32,11 @@ Landing await_piece(const uint32_t *flag, uint32_t epoch, Idle &&idle, State &&s
 }
 
 // Has the page of *p mapped for writing without changing what it holds: one
-// locked add of zero, which another thread's store cannot be lost to.
+// locked add of zero to the aligned word there, which another thread's store
+// cannot be lost to.
 inline void map_for_writing(float *p) {
-    __asm__ volatile("lock; addl $0, %0" : "+m"(*reinterpret_cast<uint32_t *>(p)) : : "cc");
+    auto *word = reinterpret_cast<uint32_t *>(reinterpret_cast<uintptr_t>(p) & ~uintptr_t{3});
+    __asm__ volatile("lock; addl $0, %0" : "+m"(*word) : : "cc");
 }
 
 }  // namespace qwn

@@ -52,6 +52,7 @@ int main() {
         float before[4];
         std::memcpy(before, page, sizeof(page));
         for (float &p : page) map_for_writing(&p);
+        for (int i = 1; i < 13; ++i) map_for_writing(reinterpret_cast<float *>(reinterpret_cast<char *>(page) + i));
         check(std::memcmp(before, page, sizeof(page)) == 0, "a page that is mapped keeps what it holds");
     }
     if (!failures) std::printf("ok\n");
