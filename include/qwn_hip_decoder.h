@@ -95,21 +95,24 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_reset(QwnCudaContextHandle *context, QwnHip
  * host) may be NULL. */
 QWN_CUDA_ABI_API int qwn_hip_decoder_forward(QwnCudaContextHandle *context, QwnHipDecoderHandle *decoder,
                                              int32_t token, float *logits, int32_t *next_token);
-/* `count` prompt tokens at the current position in prefill blocks of up to
- * 16 tokens: each projection of a block is one batched GEMV (the weights
- * are read once per block instead of once per token), then RoPE, the Q8
- * append and causal attention per token.  Same cache contents and, up to
+/* `count` prompt tokens at the current position in prefill blocks: up to 64
+ * tokens as one block, more in blocks of up to 1024 where every projection
+ * has its MFMA-order copy (else of 64).  Each projection of a block is one
+ * batched GEMM (the weights are read once per block instead of once per
+ * token), then RoPE, the Q8 append and causal attention of the block's
+ * tokens.  Same cache contents and, up to
  * the fp32 summation order of the norms, the same logits as `count`
  * forward() calls (c/qwanto_decode.c:2093 steps the prompt token by token).
- * `logits` / `next_token`: those of the last token (may be NULL). */
+ * `logits` / `next_token`: those of the last token (may be NULL; logits in
+ * host or GPU memory). */
 QWN_CUDA_ABI_API int qwn_hip_decoder_prefill(QwnCudaContextHandle *context, QwnHipDecoderHandle *decoder,
                                              const int32_t *tokens, uint32_t count, float *logits,
                                              int32_t *next_token);
 /* Speculative-decoding verification: `count` (1..16) draft tokens at the
  * current position as one block (as qwn_hip_decoder_prefill), with the tied
- * LM head run on EVERY token of the block in one batched F16 GEMV:
- * logits [count][vocab] (host, may be NULL) are the logits after each
- * token, next_tokens[count] (may be NULL) the greedy choice after each --
+ * LM head run on EVERY token of the block in one launch:
+ * logits [count][vocab] (host or GPU memory, may be NULL) are the logits after
+ * each token, next_tokens[count] (as logits) the greedy choice after each --
  * the [nodes x vocab] scores a draft-tree verifier consumes
  * (c/qwanto_jetspec.c:160-205), where the reference steps its target model
  * token by token (c/qwn_speculative.c:389-433).  The cache then holds all
@@ -125,9 +128,9 @@ QWN_CUDA_ABI_API int qwn_hip_decoder_verify(QwnCudaContextHandle *context, QwnHi
  * rotated for position P + depth(i), its K/V held
  * at cache slot P + i, and it attends to the prefix, its ancestors and
  * itself (the ancestor mask of qwn_jetspec_build_tree_mask,
- * c/qwanto_jetspec.c:33-49).  logits [count][vocab] (host, may be NULL) are
- * the target's logits after each node -- the prediction for its children --
- * and next_tokens[count] (may be NULL) their first maxima.  The rows
+ * c/qwanto_jetspec.c:33-49).  logits [count][vocab] (host or GPU memory, may
+ * be NULL) are the target's logits after each node -- the prediction for its
+ * children -- and next_tokens[count] (as logits) their first maxima.  The rows
  * qwn_jetspec_verify_tree reads (c/qwanto_jetspec.c:160-205: row i is the
  * target's prediction FOR node i) are the logits of node i's parent, or,
  * for a root, the logits after the prefix's last token.  The position stays

@@ -37,7 +37,7 @@ __device__ __forceinline__ size_t scale_index(const KvCache &c, uint32_t token, 
 }
 
 // Whether slot t is attended under a tree mask relative to slot `base`
-// (no tree: tree_bits() gives all ones).  The 64-bit test is a lookup of
+// (no tree: a base past every slot).  The 64-bit test is a lookup of
 // the mask's two halves by the slot's offset, written without any shift by
 // a wrapped offset: an earlier form, t < base || (mask >> min(t - base,
 // 63)) & 1, was compiled into the shift alone (the t < base test dropped),

@@ -70,8 +70,8 @@ ResidentKv *cache_of(Context *ctx, const QwnCudaKvCacheHandle &h) {
 // flag, after every store of the piece has reached the host's memory.  A
 // runtime copy into pageable memory pins or stages it piece by piece without
 // overlap, and one into pinned memory costs about 25 us a piece with its
-// event.  One row of 151936 logits adds 36 us to a decode step instead of 66,
-// eight rows 260 us to a verify call instead of 388.
+// event.  One row of 151936 logits adds 49 us to a decode step (72 by a
+// runtime copy), eight rows 200 us to a verify call (390).
 constexpr uint32_t kSlices = 16;
 constexpr uint32_t kSlice = kDownloadPiece / kSlices;
 __global__ __launch_bounds__(256) void download_kernel(const float *__restrict__ src, float *__restrict__ dst,
